@@ -12,6 +12,8 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -26,20 +28,20 @@ OFFLOAD_ARCH = os.environ.get("TEA_OFFLOAD_ARCH", "gfx950")
 # -ffp-contract=off: no implicit fused multiply-add, so every kernel evaluates
 # its expressions exactly as written (bitwise equal to the CPU evaluation).
 # -packed-fp32-ops: the compiler must not emit packed FP32 instructions.
-HIP_FLAGS = [
+COMPILE_FLAGS = [
     f"--offload-arch={OFFLOAD_ARCH}",
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-ffp-contract=off",
     "-fvisibility=hidden",
-    "-Wl,-soname,libtea_engine.so",
     "-Xclang",
     "-target-feature",
     "-Xclang",
     "-packed-fp32-ops",
 ]
+LINK_FLAGS = [f"--offload-arch={OFFLOAD_ARCH}", "-shared", "-fPIC", "-Wl,-soname,libtea_engine.so"]
+SOURCES = [CSRC / "engine.hip", CSRC / "warmstart.hip"]
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:
@@ -50,9 +52,14 @@ def _run(cmd: list[str], cwd: Path | None = None) -> None:
 
 
 def build_engine() -> Path:
-    sources = [CSRC / "engine.hip", CSRC / "warmstart.hip"]
+    # one object per source, compiled side by side, then linked
     tmp = ENGINE_SO.with_suffix(".so.tmp")
-    _run([HIPCC, *HIP_FLAGS, "-o", str(tmp), *map(str, sources)])
+    with tempfile.TemporaryDirectory() as folder:
+        objects = [Path(folder) / (s.stem + ".o") for s in SOURCES]
+        jobs = [[HIPCC, *COMPILE_FLAGS, "-c", str(s), "-o", str(o)] for s, o in zip(SOURCES, objects)]
+        with ThreadPoolExecutor(len(jobs)) as pool:
+            list(pool.map(_run, jobs))
+        _run([HIPCC, *LINK_FLAGS, "-o", str(tmp), *map(str, objects)])
     os.replace(tmp, ENGINE_SO)
     return ENGINE_SO
 

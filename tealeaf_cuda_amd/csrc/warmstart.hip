@@ -15,6 +15,7 @@
 // permutation of K inside the hardware leaves the product unchanged.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -31,6 +32,7 @@ namespace ws {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+typedef __attribute__((__vector_size__(4 * sizeof(unsigned int)))) unsigned int uintx4;
 
 constexpr int BLOCK = 256;
 constexpr int NPLANES = 6;   // training sample: f0, f1, f2, target, Kx, Ky
@@ -659,109 +661,223 @@ __global__ void k_out_bwd(const float *__restrict__ g6, const float *__restrict_
     }
 }
 
-// Layer 6 weight and bias gradients: thread j < 288 owns W6[tap][ci], thread
-// 288 owns b6; workgroup c sums pixels [c*n/chunks, (c+1)*n/chunks).
-constexpr int OUT_WG_THREADS = 320;
-__global__ __launch_bounds__(OUT_WG_THREADS) void k_out_wgrad(const __bf16 *__restrict__ a5,
-                                                               const float *__restrict__ g6, float *__restrict__ part,
-                                                               int B, int H, int W, int chunks)
+// Workgroups of a weight-gradient reduction: each sums its share of the pixels
+// in registers and writes one partial, which k_sum_parts adds in a fixed order.
+// 512 (two per compute unit) keeps the partials at 19 MB per layer.
+constexpr int WG_PARTS = 512;
+
+// Layer 6 weight and bias gradients, dW6[tap][ci] = sum_p a5[p + tap][ci] g6[p]
+// and db6 = sum_p g6[p], summed over the input pixels q = p + tap (a5 and g6
+// are zero on the border).  One product per 72 loaded values, so the pass is
+// bound by reading a5 once: a lane holds 8 channels of one pixel column
+// (one 16-byte load per pixel), marches down a run of rows and keeps the 3x3
+// window of g6 and the 72 sums in registers; 4 lanes cover a pixel, a wave 16
+// columns.  32 x 128 x 128 pixels: 1060 us with one thread per weight walking
+// every pixel, 20 us here.  tasks: (image, 16 columns, run of rows).
+__global__ __launch_bounds__(BLOCK) void k_out_wgrad(const __bf16 *__restrict__ a5, const float *__restrict__ g6,
+                                                     float *__restrict__ part, int H, int W, int rows, int nruns,
+                                                     long tasks)
 {
-    const int j = threadIdx.x;
-    if (j > TAPS * CH) return;
-    const long n = (long)B * H * W;
-    const long p0 = n * blockIdx.x / chunks, p1 = n * (blockIdx.x + 1) / chunks;
-    const int t = j / CH, ci = j % CH;
-    float acc = 0.0f;
-    for (long p = p0; p < p1; p++) {
-        const int x = (int)(p % W), y = (int)((p / W) % H), b = (int)(p / ((long)W * H));
-        const float g = g6[padded(b, y, x, H, W)];
-        if (j == TAPS * CH) acc += g;
-        else acc += (float)a5[padded(b, y + t / 3 - 1, x + t % 3 - 1, H, W) * CH + ci] * g;
+    constexpr int NOUT = TAPS * CH + 1, NW = BLOCK / 64;
+    __shared__ float lds[NW][NOUT];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q = lane & 3, px = lane >> 2;
+    const int cols = W / 16;
+    float acc[TAPS][8], accb = 0.0f;
+#pragma unroll
+    for (int t = 0; t < TAPS; t++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) acc[t][i] = 0.0f;
+    for (long task = (long)blockIdx.x * NW + wave; task < tasks; task += (long)gridDim.x * NW) {
+        const int run = (int)(task % nruns);
+        const int xg = (int)((task / nruns) % cols), b = (int)(task / nruns / cols);
+        const int x = xg * 16 + px, y0 = run * rows, y1 = min(y0 + rows, H);
+        // gw[k][j] = g6 at row y - 1 + k, column x - 1 + j
+        float gw[3][3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            gw[1][j] = g6[padded(b, y0 - 1, x - 1 + j, H, W)];
+            gw[2][j] = g6[padded(b, y0, x - 1 + j, H, W)];
+        }
+        for (int y = y0; y < y1; y++) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                gw[0][j] = gw[1][j];
+                gw[1][j] = gw[2][j];
+                gw[2][j] = g6[padded(b, y + 1, x - 1 + j, H, W)];
+            }
+            const bf16x8 a = *(const bf16x8 *)(a5 + padded(b, y, x, H, W) * CH + q * 8);
+            accb += gw[1][1];
+#pragma unroll
+            for (int t = 0; t < TAPS; t++) {
+                const float g = gw[2 - t / 3][2 - t % 3];   // g6 at p = q - tap
+#pragma unroll
+                for (int i = 0; i < 8; i++) acc[t][i] += (float)a[i] * g;
+            }
+        }
     }
-    part[(long)blockIdx.x * (TAPS * CH + 1) + j] = acc;
+#pragma unroll
+    for (int off = 32; off >= 4; off >>= 1) {
+#pragma unroll
+        for (int t = 0; t < TAPS; t++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) acc[t][i] += __shfl_xor(acc[t][i], off, 64);
+        accb += __shfl_xor(accb, off, 64);
+    }
+    if (px == 0) {
+#pragma unroll
+        for (int t = 0; t < TAPS; t++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) lds[wave][t * CH + q * 8 + i] = acc[t][i];
+        if (q == 0) lds[wave][TAPS * CH] = accb;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < NOUT; e += BLOCK)
+        part[(long)blockIdx.x * NOUT + e] = (lds[0][e] + lds[1][e]) + (lds[2][e] + lds[3][e]);
 }
 
-// Weight gradient of a 32-channel layer: dW[tap][ci][co] = sum_p in[p + tap][ci] * g[p][co],
-// pixels in groups of 32 along a row (K of one MFMA).  Grid (NTAP, chunks),
-// 4 waves per workgroup taking every 4th group of the workgroup's range; the
-// workgroup's 32x32 sum goes to part[chunk][tap][ci][co].
+// Weight and bias gradients of a 32-channel layer: dW[tap][ci][co] =
+// sum_q in[q][ci] g[q - tap][co] over the input pixels q (both images are zero
+// on the border) and db[co] = sum_p g[p][co], as products with K = 32 pixels of
+// a row on the matrix cores.  Both operands need 8 consecutive pixels of one
+// channel per lane, across the images' layout, so rows are turned on their way
+// into LDS ([channel][pixel], pixels in pairs: one 4-byte store per two) and
+// each staged row serves all nine taps: `in` rows meet a ring of g rows, and the
+// left and right taps come from the centre fragment by funnel shifts.  A
+// workgroup marches down a run of rows of a 64-pixel band, two rows per step;
+// wave (cb, nb) owns one 16 x 16 block of every tap, so no sums cross waves,
+// and the bias is a tenth product with a row of ones.  Reading the two images
+// once is the floor (13 us at 32 x 128 x 128); one workgroup per tap gathering
+// 2-byte values took 82 us and the bias alone 132 us, this takes 29 us for both.
+// NTAP = 1: the im2col image of layer 1 (27 of 32 rows kept, centre tap only).
+constexpr int WGR_IN = 36, WGR_G = 44;   // 4-byte words per channel row: 16-byte aligned rows, spread over the banks
+constexpr int WGR_G0 = 8;                // index of the band's first pixel in a g row
 template <int NTAP>
 __global__ __launch_bounds__(BLOCK) void k_wgrad32(const __bf16 *__restrict__ in, const __bf16 *__restrict__ g,
-                                                   float *__restrict__ part, int B, int H, int W, int chunks)
+                                                   float *__restrict__ part, int H, int W, int rows, int nruns,
+                                                   long tasks)
 {
-    __shared__ float lds[4][CH * CH];
+    constexpr int NIN = NTAP == 1 ? K1 : CH, NPART = NTAP * NIN * CH + CH;
+    constexpr int RING = 4;   // g rows y - 1 .. y + 2 of a step
+    __shared__ __attribute__((aligned(16))) unsigned int tin[2][CH * WGR_IN];
+    __shared__ __attribute__((aligned(16))) unsigned int tg[RING][CH * WGR_G];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m = lane & 15, kg = lane >> 4;
-    const int t = blockIdx.x, c = blockIdx.y;
-    const int dy = NTAP == 1 ? 0 : t / 3 - 1, dx = NTAP == 1 ? 0 : t % 3 - 1;
-    const long groups = (long)B * H * W / 32;
-    const long g0 = groups * c / chunks, g1 = groups * (c + 1) / chunks;
-    floatx4 acc[2][2];
+    const int m = lane & 15, kg = lane >> 4, cb = wave >> 1, nb = wave & 1;
+    const int bands = W / 64;
+    // two pixels x 8 channels of a row, px and px + 1 (each inside the padded
+    // row or zero), to word `word` of the 8 channel rows
+    auto turn = [&](const __bf16 *img, int b, int y, int x0, int px, int lo, int hi, int q8, unsigned int *dst,
+                    int stride, int word) {
+        uintx4 v[2];   // channels 2j, 2j + 1 of a pixel in word j
 #pragma unroll
-    for (int i = 0; i < 2; i++) acc[i][0] = acc[i][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (long gi = g0 + wave; gi < g1; gi += 4) {
-        const long p0 = gi * 32;
-        const int b = (int)(p0 / ((long)W * H));
-        const int rem = (int)(p0 % ((long)W * H));
-        const int y = rem / W, xg = rem % W;
-        bf16x8 av[2], gv[2];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int xk = xg + kg * 8 + i;
-            const long pa = padded(b, y + dy, xk + dx, H, W) * CH;
-            const long pg = padded(b, y, xk, H, W) * CH;
-            av[0][i] = in[pa + m];
-            av[1][i] = in[pa + 16 + m];
-            gv[0][i] = g[pg + m];
-            gv[1][i] = g[pg + 16 + m];
+        for (int k = 0; k < 2; k++) {
+            v[k] = uintx4{0, 0, 0, 0};
+            if (px + k >= lo && px + k <= hi && y <= H)
+                v[k] = *(const uintx4 *)(img + padded(b, y, x0 + px + k, H, W) * CH + q8 * 8);
         }
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++) {
-            acc[cb][0] = mfma(av[cb], gv[0], acc[cb][0]);
-            acc[cb][1] = mfma(av[cb], gv[1], acc[cb][1]);
+        for (int j = 0; j < 4; j++) {
+            dst[(q8 * 8 + 2 * j) * stride + word] = (v[0][j] & 0xffffu) | (v[1][j] << 16);
+            dst[(q8 * 8 + 2 * j + 1) * stride + word] = (v[0][j] >> 16) | (v[1][j] & 0xffff0000u);
+        }
+    };
+    auto stage_in = [&](int b, int y, int x0, unsigned int *dst, int t0) {
+        for (int e = t0; e < 32 * 4; e += BLOCK / 2) turn(in, b, y, x0, (e >> 2) * 2, 0, 63, e & 3, dst, WGR_IN, e >> 2);
+    };
+    auto stage_g = [&](int b, int y, int x0, unsigned int *dst, int t0) {   // pixels -1 .. 64
+        for (int e = t0; e < 34 * 4; e += BLOCK / 2)
+            turn(g, b, y, x0, (e >> 2) * 2 - 2, -1, 64, e & 3, dst, WGR_G, WGR_G0 / 2 - 1 + (e >> 2));
+    };
+    floatx4 acc[NTAP], accb = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < NTAP; t++) acc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; i++) ones[i] = (__bf16)1.0f;
+    const int half = threadIdx.x / (BLOCK / 2), t0 = threadIdx.x % (BLOCK / 2);
+    for (long task = blockIdx.x; task < tasks; task += gridDim.x) {
+        const int run = (int)(task % nruns);
+        const int band = (int)((task / nruns) % bands), b = (int)(task / nruns / bands);
+        const int x0 = band * 64, y0 = run * rows, y1 = min(y0 + rows, H);
+        __syncthreads();   // the last task's reads are done
+        if (NTAP > 1) stage_g(b, y0 - 1 + half, x0, tg[(y0 - 1 + half + RING) % RING], t0);
+        for (int y = y0; y < y1; y += 2) {
+            stage_in(b, y + half, x0, tin[half], t0);
+            const int yg = NTAP > 1 ? y + 1 + half : y + half;
+            stage_g(b, yg, x0, tg[yg % RING], t0);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                if (y + k >= y1) continue;
+#pragma unroll
+                for (int grp = 0; grp < 2; grp++) {
+                    const int px = grp * 32 + kg * 8;
+                    const bf16x8 av =
+                        __builtin_bit_cast(bf16x8, *(const uintx4 *)&tin[k][(cb * 16 + m) * WGR_IN + px / 2]);
+#pragma unroll
+                    for (int dy = NTAP > 1 ? -1 : 0; dy <= (NTAP > 1 ? 1 : 0); dy++) {
+                        // tap row dy + 1 meets g row y - dy
+                        const unsigned int *gr =
+                            &tg[(y + k - dy + RING) % RING][(nb * 16 + m) * WGR_G + (WGR_G0 + px) / 2];
+                        const uintx4 w = *(const uintx4 *)gr;
+                        const bf16x8 gc = __builtin_bit_cast(bf16x8, w);
+                        if (NTAP == 1) {
+                            acc[0] = mfma(av, gc, acc[0]);
+                        } else {
+                            // dx = 1 takes g one pixel to the left, dx = -1 one to the right
+                            const unsigned int wl = gr[-1], wr = gr[4];
+                            uintx4 l, r;
+                            l[0] = __builtin_amdgcn_alignbit(w[0], wl, 16);
+                            l[1] = __builtin_amdgcn_alignbit(w[1], w[0], 16);
+                            l[2] = __builtin_amdgcn_alignbit(w[2], w[1], 16);
+                            l[3] = __builtin_amdgcn_alignbit(w[3], w[2], 16);
+                            r[0] = l[1];
+                            r[1] = l[2];
+                            r[2] = l[3];
+                            r[3] = __builtin_amdgcn_alignbit(wr, w[3], 16);
+                            const int t = (dy + 1) * 3;
+                            acc[t % NTAP] = mfma(av, __builtin_bit_cast(bf16x8, r), acc[t % NTAP]);
+                            acc[(t + 1) % NTAP] = mfma(av, gc, acc[(t + 1) % NTAP]);
+                            acc[(t + 2) % NTAP] = mfma(av, __builtin_bit_cast(bf16x8, l), acc[(t + 2) % NTAP]);
+                        }
+                        if (dy == 0 && cb == 0) accb = mfma(ones, gc, accb);
+                    }
+                }
+            }
+            __syncthreads();
         }
     }
+    float *dst = part + (long)blockIdx.x * NPART;
 #pragma unroll
-    for (int cb = 0; cb < 2; cb++)
+    for (int t = 0; t < NTAP; t++)
 #pragma unroll
-        for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) lds[wave][(cb * 16 + kg * 4 + i) * CH + nb * 16 + m] = acc[cb][nb][i];
-    __syncthreads();
-    float *dst = part + ((long)c * NTAP + t) * CH * CH;
-    for (int e = threadIdx.x; e < CH * CH; e += BLOCK) dst[e] = lds[0][e] + lds[1][e] + lds[2][e] + lds[3][e];
+        for (int i = 0; i < 4; i++) {
+            const int ci = cb * 16 + kg * 4 + i;
+            if (ci < NIN) dst[(t * NIN + ci) * CH + nb * 16 + m] = acc[t][i];
+        }
+    if (cb == 0 && kg == 0) dst[NTAP * NIN * CH + nb * 16 + m] = accb[0];
 }
 
-// Bias gradient of a 32-channel layer: per-workgroup channel sums of g.
-__global__ __launch_bounds__(BLOCK) void k_chansum(const __bf16 *__restrict__ g, float *__restrict__ part, int B,
-                                                   int H, int W, int chunks)
+// dst[e] = sum_c part[c*n + e], e < n (fixed order): 32 consecutive e per
+// workgroup, every 8th partial per thread, then the 8 sums in order.  Bound by
+// reading the partials; one thread walking all of them took 58 us for 256 x
+// 9216 values, this takes 5 us for 512 x 9248.
+__global__ __launch_bounds__(BLOCK) void k_sum_parts(const float *__restrict__ part, int chunks, int n,
+                                                     float *__restrict__ dst)
 {
-    __shared__ float lds[BLOCK];
-    const int co = threadIdx.x % CH, sub = threadIdx.x / CH;
-    const long n = (long)B * H * W;
-    const long p0 = n * blockIdx.x / chunks, p1 = n * (blockIdx.x + 1) / chunks;
-    float acc = 0.0f;
-    for (long p = p0 + sub; p < p1; p += BLOCK / CH) {
-        const int x = (int)(p % W), y = (int)((p / W) % H), b = (int)(p / ((long)W * H));
-        acc += (float)g[padded(b, y, x, H, W) * CH + co];
-    }
-    lds[threadIdx.x] = acc;
-    __syncthreads();
-    if (threadIdx.x < CH) {
-        float s = 0.0f;
-        for (int k = 0; k < BLOCK / CH; k++) s += lds[k * CH + threadIdx.x];
-        part[(long)blockIdx.x * CH + threadIdx.x] = s;
-    }
-}
-
-// dst[e] = sum_c part[c*stride + e], e < n (fixed order).
-__global__ void k_sum_parts(const float *__restrict__ part, long stride, int chunks, int n, float *__restrict__ dst)
-{
-    const int e = blockIdx.x * BLOCK + threadIdx.x;
-    if (e >= n) return;
+    __shared__ float lds[BLOCK / 32][32];
+    const int k = threadIdx.x & 31, sub = threadIdx.x >> 5, e = blockIdx.x * 32 + k;
     float s = 0.0f;
-    for (int c = 0; c < chunks; c++) s += part[(long)c * stride + e];
-    dst[e] = s;
+    if (e < n) {
+#pragma unroll 8
+        for (int c = sub; c < chunks; c += BLOCK / 32) s += part[(long)c * n + e];
+    }
+    lds[sub][k] = s;
+    __syncthreads();
+    if (sub == 0 && e < n) {
+        for (int j = 1; j < BLOCK / 32; j++) s += lds[j][k];
+        dst[e] = s;
+    }
 }
 
 // Adam (Kingma and Ba, 2015) on the FP32 master parameters.
@@ -998,8 +1114,6 @@ int ws_fail(const char *fmt, ...)
         if (e_ != hipSuccess) return ws_fail("%s: %s", #call, hipGetErrorString(e_));  \
     } while (0)
 
-constexpr int WG_CHUNKS = 256;      // workgroups per weight-gradient reduction
-
 struct Trainer {
     int B = 0, H = 0, W = 0, margin = 0, energy = 0;
     long step = 0;
@@ -1035,6 +1149,11 @@ int forward_pass(Trainer *t, const float *samples)
     return 0;
 }
 
+void sum_parts(const float *part, int parts, int n, float *dst, hipStream_t s)
+{
+    hipLaunchKernelGGL(ws::k_sum_parts, dim3((n + 31) / 32), dim3(ws::BLOCK), 0, s, part, parts, n, dst);
+}
+
 // loss, then every gradient into t->grad (same layout as the parameters)
 int backward_pass(Trainer *t, const float *samples)
 {
@@ -1047,25 +1166,35 @@ int backward_pass(Trainer *t, const float *samples)
     hipLaunchKernelGGL(k_loss, dim3(t->loss_blocks), dim3(BLOCK), 0, s, t->acts.out, samples, t->g6, t->loss_part,
                        B, H, W, t->margin, scale, t->energy);
     // layer 6
-    hipLaunchKernelGGL(k_out_wgrad, dim3(WG_CHUNKS), dim3(OUT_WG_THREADS), 0, s, t->acts.a[5], t->g6, t->part, B,
-                       H, W, WG_CHUNKS);
-    hipLaunchKernelGGL(k_sum_parts, dim3(nblocks(TAPS * CH + 1)), dim3(BLOCK), 0, s, t->part,
-                       (long)(TAPS * CH + 1), WG_CHUNKS, TAPS * CH + 1, t->grad + OFF_W6);
+    {
+        // about 2048 waves; a run no shorter than 8 rows (two more are read for the window)
+        const long cols = (long)B * (W / 16);
+        const int rows = (int)std::min<long>(H, std::max<long>(8, (cols * H + 2047) / 2048));
+        const int nruns = (H + rows - 1) / rows;
+        const long tasks = cols * nruns;
+        const int parts = (int)std::min<long>(WG_PARTS, (tasks + 3) / 4);
+        hipLaunchKernelGGL(k_out_wgrad, dim3(parts), dim3(BLOCK), 0, s, t->acts.a[5], t->g6, t->part, H, W, rows,
+                           nruns, tasks);
+        sum_parts(t->part, parts, TAPS * CH + 1, t->grad + OFF_W6, s);
+    }
     hipLaunchKernelGGL(k_out_bwd, dim3(nblocks(npix)), dim3(BLOCK), 0, s, t->g6, t->net.w6, t->acts.a[5], t->g[0],
                        B, H, W);
+    // the 32-channel layers: two workgroups per compute unit, runs of an even number of rows (two per step),
+    // no shorter than 8 (the run's g rows above and below are read twice)
+    const long bands = (long)B * (W / 64);
+    const int wrows = (int)std::min<long>(H, std::max<long>(8, (bands * H + WG_PARTS - 1) / WG_PARTS + 1) & ~1L);
+    const int wruns = (H + wrows - 1) / wrows;
+    const int wparts = (int)std::min<long>(WG_PARTS, bands * wruns);
     // layers 5..2: weight and bias gradients from g(l), then g(l-1)
     const int rows = conv_rows(H);
     const dim3 grid(W / 64, H / rows, B), block(rows * 64);
     const bf16x8 *pk = (const bf16x8 *)t->net.packed;
     int cur = 0;
     for (int l = 5; l >= 2; l--) {
-        hipLaunchKernelGGL((k_wgrad32<TAPS>), dim3(TAPS, WG_CHUNKS), dim3(BLOCK), 0, s, t->acts.a[l - 1], t->g[cur],
-                           t->part, B, H, W, WG_CHUNKS);
-        hipLaunchKernelGGL(k_sum_parts, dim3(nblocks(TAPS * CH * CH)), dim3(BLOCK), 0, s, t->part,
-                           (long)TAPS * CH * CH, WG_CHUNKS, TAPS * CH * CH, t->grad + off_w(l));
-        hipLaunchKernelGGL(k_chansum, dim3(WG_CHUNKS), dim3(BLOCK), 0, s, t->g[cur], t->part, B, H, W, WG_CHUNKS);
-        hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(BLOCK), 0, s, t->part, (long)CH, WG_CHUNKS, CH,
-                           t->grad + off_b(l));
+        // weights and bias are neighbours in the parameter vector
+        hipLaunchKernelGGL((k_wgrad32<TAPS>), dim3(wparts), dim3(BLOCK), 0, s, t->acts.a[l - 1], t->g[cur], t->part,
+                           H, W, wrows, wruns, bands * wruns);
+        sum_parts(t->part, wparts, HID_SIZE, t->grad + off_w(l), s);
         if (rows == 8)
             hipLaunchKernelGGL((k_conv32<8, true>), grid, block, 0, s, t->g[cur], t->g[1 - cur], pk + pk_bwd(l) / 8,
                                (const float *)nullptr, t->acts.a[l - 1], H, W);
@@ -1075,12 +1204,9 @@ int backward_pass(Trainer *t, const float *samples)
         cur = 1 - cur;
     }
     // layer 1 (im2col input, no input gradient)
-    hipLaunchKernelGGL((k_wgrad32<1>), dim3(1, WG_CHUNKS), dim3(BLOCK), 0, s, t->acts.x1, t->g[cur], t->part, B, H,
-                       W, WG_CHUNKS);
-    hipLaunchKernelGGL(k_sum_parts, dim3(nblocks(K1 * CH)), dim3(BLOCK), 0, s, t->part, (long)CH * CH, WG_CHUNKS,
-                       K1 * CH, t->grad + OFF_W1);
-    hipLaunchKernelGGL(k_chansum, dim3(WG_CHUNKS), dim3(BLOCK), 0, s, t->g[cur], t->part, B, H, W, WG_CHUNKS);
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(BLOCK), 0, s, t->part, (long)CH, WG_CHUNKS, CH, t->grad + OFF_B1);
+    hipLaunchKernelGGL((k_wgrad32<1>), dim3(wparts), dim3(BLOCK), 0, s, t->acts.x1, t->g[cur], t->part, H, W, wrows,
+                       wruns, bands * wruns);
+    sum_parts(t->part, wparts, K1 * CH + CH, t->grad + OFF_W1, s);
     WS_OK(hipGetLastError());
     return 0;
 }
@@ -1129,7 +1255,7 @@ EXPORT void *tea_ws_trainer_create(int batch, int height, int width, int margin,
     t->loss_blocks = (int)ws::nblocks(npix);
     const size_t gbytes = ws::act_bytes(batch, height, width);
     const size_t g6bytes = (size_t)batch * (height + 2) * (width + 2) * sizeof(float);
-    const size_t part_floats = (size_t)WG_CHUNKS * ws::TAPS * ws::CH * ws::CH;
+    const size_t part_floats = (size_t)ws::WG_PARTS * ws::HID_SIZE;
     bool ok = hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking) == hipSuccess &&
               ws::net_alloc(t->net) == hipSuccess && ws::acts_alloc(t->acts, batch, height, width, true) == hipSuccess &&
               hipMalloc(&t->g6, g6bytes) == hipSuccess && hipMemset(t->g6, 0, g6bytes) == hipSuccess &&
