@@ -264,6 +264,38 @@ void tea_engine_ppcg_iteration(int with_p, double beta, double theta, int inner_
  * boundaries (the reference driver's update_halo of p between calc_p and
  * calc_w is a no-op there). */
 void tea_engine_cg_begin_ur(int with_p, double beta, double rro, double *pw, double *rrn);
+/* A run of tea_engine_cg_begin_ur calls in one launch, for meshes whose fields
+ * stay on the chip: the first as given, each later one with_p, beta = rrn / rro
+ * and rro = rrn of the one before.  The run ends after max_its calls, after
+ * 1024, or after the first for which one of the caller's tests holds:
+ *   sqrt|rrn| < stop[0];
+ *   it is call stop[1] of the run or a later one, and sqrt|rrn| <= stop[2];
+ *   stop[3] != 0 (residual replacement): with drop = sqrt|rrn / q_ref|,
+ *   not (drop >= stop[7] and sqrt|stop[6]| * drop >= stop[8]), where q_ref is
+ *   stop[5], or with stop[4] == 0 the first rrn of the run (not tested itself).
+ * pw[k] and rrn[k] are call k's values.  Returns the calls made; 0 when the
+ * mesh does not fit or not all of the chip is free (nothing was done: make the
+ * calls one by one). */
+int tea_engine_cg_run(int with_p, double beta, double rro, int max_its, const double *stop, double *pw, double *rrn);
+/* The same for PPCG outer iterations (zero-flux boundaries: the fields' halo
+ * cells outside the mesh are taken as 0 where they meet a face coefficient):
+ * tea_engine_ppcg_begin_ur(with_p, beta, theta), inner steps 1..inner_steps,
+ * tea_engine_ppcg_end, then the next with with_p and beta = the end's r.z over
+ * the begin's.  With from_inner the run first completes an iteration whose ur
+ * has been done and whose r may have been replaced since: z = M^-1 r,
+ * ppcg_init_sd_new(theta), the inner steps, the end (beta = its r.z / rro).
+ * values[4k ..] are p.w, r.z, ur's r.z and the end's r.z of iteration k.
+ * stop[0] is tested on the end's value, stop[3..8] on ur's: when that test
+ * ends the run, *at_ur = 1 and the last iteration stops after its ur (its
+ * values[3] is 0).  *rrn_end: the latest end's value.  stop[1..2] are not
+ * used.  Returns the iterations begun; 0 as for tea_engine_cg_run. */
+int tea_engine_ppcg_run(int from_inner, int with_p, double beta, double rro, double theta, int inner_steps,
+                        int max_its, const double *stop, double *values, int *at_ur, double *rrn_end);
+/* And for Chebyshev iterations step, step + 1, ..., numbered n, n + 1, ... by
+ * the caller: after those with number >= check_from that ten divides, error is
+ * the r.r of tea_leaf_calc_2norm_kernel_cuda_ (rr[k]; else rr[k] = 0); after
+ * each, error becomes sqrt|error|, and the run ends when that is below target. */
+int tea_engine_cheby_run(int step, int n, int check_from, double error, double target, int max_its, double *rr);
 /* ---- Chebyshev iterations in passes ------------------------------------------- *
  * No counterpart in the reference: tea_leaf_cheby_iterate_kernel_cuda_ for
  * cheby_calc_step = step .. step + nsteps - 1 (tea_leaf_kernel_cuda.cu:125-135),

@@ -861,6 +861,37 @@ EXPORT void tea_engine_cg_begin_ur(int with_p, double beta, double rro, double *
     tea_leaf_cg_calc_ur_kernel_cuda_(&alpha, rrn);
 }
 
+/* the run's own tests, shared with the PPCG run */
+static int run_stops(int call, double rrn, const double *stop, double *q_ref, int *have_q)
+{
+    int end = sqrt(fabs(rrn)) < stop[0] || (call >= (int)stop[1] && sqrt(fabs(rrn)) <= stop[2]);
+    if (stop[3] != 0.0) {
+        if (!*have_q) {
+            *q_ref = rrn;
+            *have_q = 1;
+        } else {
+            const double drop = sqrt(fabs(rrn / *q_ref));
+            end = end || !(drop >= stop[7] && sqrt(fabs(stop[6])) * drop >= stop[8]);
+        }
+    }
+    return end;
+}
+
+EXPORT int tea_engine_cg_run(int with_p, double beta, double rro, int max_its, const double *stop, double *pw,
+                             double *rrn)
+{
+    double q_ref = stop[5];
+    int have_q = stop[4] != 0.0, k;
+    for (k = 0; k < max_its && k < 1024; k++) {
+        tea_engine_cg_begin_ur(with_p, beta, rro, &pw[k], &rrn[k]);
+        if (run_stops(k + 1, rrn[k], stop, &q_ref, &have_q)) return k + 1;
+        with_p = 1;
+        beta = rrn[k] / rro;
+        rro = rrn[k];
+    }
+    return k;
+}
+
 EXPORT void tea_engine_ppcg_end(double *rrn);
 EXPORT void tea_engine_ppcg_end_begin_ur(double rro_prev, double theta, double *rrn_end, double *pw_rro,
                                          double *rrn)
@@ -890,6 +921,59 @@ EXPORT void tea_engine_ppcg_iteration(int with_p, double beta, double theta, int
     tea_engine_ppcg_begin_ur(with_p, beta, theta, pw_rro, rrn_ur);
     if (inner_steps > 0) tea_engine_ppcg_inner_n(1, inner_steps);
     tea_engine_ppcg_end(rrn_end);
+}
+
+EXPORT void tea_engine_ppcg_inner_n(int step, int nsteps);
+EXPORT int tea_engine_ppcg_run(int from_inner, int with_p, double beta, double rro, double theta, int inner_steps,
+                               int max_its, const double *stop, double *values, int *at_ur, double *rrn_end)
+{
+    double q_ref = stop[5];
+    int have_q = stop[4] != 0.0, k;
+    *at_ur = 0;
+    if (from_inner) {
+        int two = 2;
+        double unused;
+        tea_leaf_ppcg_init_kernel_cuda_(&two, &unused);
+        tea_leaf_ppcg_init_sd_new_kernel_cuda_(&theta);
+        for (int s = 1; s <= inner_steps; s++) tea_engine_ppcg_inner_n(s, 1);
+        tea_engine_ppcg_end(rrn_end);
+        with_p = 1;
+        beta = *rrn_end / rro;
+    }
+    const double ur_only[9] = {-1.0, 1e9, -1.0, stop[3], 0.0, 0.0, stop[6], stop[7], stop[8]};
+    for (k = 0; k < max_its && k < 1024; k++) {
+        double *v = values + 4 * k;
+        tea_engine_ppcg_begin_ur(with_p, beta, theta, v, &v[2]);
+        v[3] = 0.0;
+        if (run_stops(k + 1, v[2], ur_only, &q_ref, &have_q)) {
+            *at_ur = 1;
+            return k + 1;
+        }
+        for (int s = 1; s <= inner_steps; s++) tea_engine_ppcg_inner_n(s, 1);
+        tea_engine_ppcg_end(rrn_end);
+        v[3] = *rrn_end;
+        if (sqrt(fabs(v[3])) < stop[0]) return k + 1;
+        with_p = 1;
+        beta = v[3] / v[1];
+    }
+    return k;
+}
+
+EXPORT int tea_engine_cheby_run(int step, int n, int check_from, double error, double target, int max_its, double *rr)
+{
+    int k;
+    for (k = 0; k < max_its && k < 1024; k++) {
+        int s = step + k, one = 1;
+        tea_leaf_cheby_iterate_kernel_cuda_(&s);
+        rr[k] = 0.0;
+        if (n + k >= check_from && (n + k) % 10 == 0) {
+            tea_leaf_calc_2norm_kernel_cuda_(&one, &error);
+            rr[k] = error;
+        }
+        error = sqrt(fabs(error));
+        if (fabs(error) < target) return k + 1;
+    }
+    return k;
 }
 
 EXPORT void tea_engine_ppcg_inner_n(int step, int nsteps)

@@ -41,7 +41,7 @@ COMPILE_FLAGS = [
     "-packed-fp32-ops",
 ]
 LINK_FLAGS = [f"--offload-arch={OFFLOAD_ARCH}", "-shared", "-fPIC", "-Wl,-soname,libtea_engine.so"]
-SOURCES = [CSRC / "engine.hip", CSRC / "warmstart.hip"]
+SOURCES = [CSRC / "engine.hip", CSRC / "resident.hip", CSRC / "warmstart.hip"]
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:

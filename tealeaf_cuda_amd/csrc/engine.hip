@@ -31,6 +31,7 @@
 #include "../../include/tea_leaf_engine.h"
 #include "engine_device.hpp"
 #include "engine_solver.hpp"
+#include "resident.hpp"
 #include "ws_net.hpp"
 
 using namespace tea;
@@ -133,6 +134,8 @@ void Profiler::drain(bool wait)
     pending.erase(pending.begin(), pending.begin() + (long)k);
 }
 
+constexpr int RUN_VALUES = 4;   // values an iteration of a resident run returns, at most
+
 struct Chunk {
     bool initialised = false;
     int nx = 0, ny = 0, h = 0;
@@ -187,6 +190,14 @@ struct Chunk {
     int end_slot = -1;
     int max_blocks = 0;              // largest grid of any launch
     int last_grid = 0;               // grid of the latest launch
+
+    // resident runs: exchange words (in the field slab), the latest tag, and
+    // the values of a run's iterations (pinned, behind h_out)
+    res::Exchange res_x{};
+    double *h_run = nullptr, *d_run = nullptr;
+    double *h_coef = nullptr, *res_coef = nullptr;   // iteration coefficients: pinned staging, device copy
+    int res_coef_at = -1, res_coef_n = 0;            // the ones the device copy holds
+    bool res_busy = false;   // a run found part of the chip taken: no more of them (finding out costs 0.2 s)
 
     double *d_halo_buf = nullptr;    // staging for pack / unpack
     size_t halo_buf_elems = 0;
@@ -1123,8 +1134,19 @@ EXPORT void initialise_cuda_(int *x_min, int *x_max, int *y_min, int *y_max)
     HIP_OK(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
     const size_t field_elems = (size_t)g.pitch * (size_t)g.rows + 16;  // + slack, keeps 128-byte alignment
     const size_t field_stride = (field_elems + 31) / 32 * 32;
-    HIP_OK(hipMalloc(&g.slab, field_stride * N_SLOTS * sizeof(double)));
-    HIP_OK(hipMemsetAsync(g.slab, 0, field_stride * N_SLOTS * sizeof(double), g.stream));
+    // behind the fields: the exchange words of resident runs (they start at zero too) and coefficients
+    const size_t slab_elems = field_stride * N_SLOTS + res::EXCHANGE_WORDS + (2 + RUN_VALUES) * res::RES_HISTORY;
+    HIP_OK(hipMalloc(&g.slab, slab_elems * sizeof(double)));
+    HIP_OK(hipMemsetAsync(g.slab, 0, slab_elems * sizeof(double), g.stream));
+    {
+        res::word_t *words = (res::word_t *)(g.slab + field_stride * N_SLOTS);
+        g.res_x.ctl = (unsigned *)words;
+        g.res_x.red = words + 16;
+        g.res_x.col = g.res_x.red + res::RED_WORDS;
+        g.res_x.row = g.res_x.col + res::COL_WORDS;
+        g.res_coef = (double *)(words + res::EXCHANGE_WORDS);
+        g.res_x.history = g.res_coef + 2 * res::RES_HISTORY;
+    }
     for (int k = 1; k < N_SLOTS; k++) {
         g.f[k] = g.slab + field_stride * k;
         g.fs[k] = g.f[k] + (g.lead - g.h);
@@ -1141,8 +1163,12 @@ EXPORT void initialise_cuda_(int *x_min, int *x_max, int *y_min, int *y_max)
         g.max_blocks = (all < grid_max() ? all : grid_max()) + 1;
     }
     HIP_OK(hipMalloc(&g.d_partials, (size_t)MAX_RED * g.max_blocks * sizeof(DD)));
-    HIP_OK(hipHostMalloc(&g.h_out, MAX_RED * sizeof(double), hipHostMallocDefault));
+    HIP_OK(hipHostMalloc(&g.h_out, (MAX_RED + 4 + (RUN_VALUES + 2) * res::RES_HISTORY) * sizeof(double),
+                         hipHostMallocDefault));
     HIP_OK(hipHostGetDevicePointer((void **)&g.d_out, g.h_out, 0));
+    g.h_run = g.h_out + MAX_RED;
+    g.d_run = g.d_out + MAX_RED;
+    g.h_coef = g.h_run + 4 + RUN_VALUES * res::RES_HISTORY;
     HIP_OK(hipMalloc(&g.d_scal, MAX_RED * sizeof(double)));
     if (!g.ev_scal) HIP_OK(hipEventCreateWithFlags(&g.ev_scal, hipEventDisableTiming));
 
@@ -2380,6 +2406,7 @@ namespace {
 void upload_coefs(const double *a, const double *b, int n)
 {
     if (n < 0) n = 0;
+    g.res_coef_at = -1;
     g.ch_a.assign(a, a + n);
     g.ch_b.assign(b, b + n);
 }
@@ -2691,6 +2718,239 @@ EXPORT void tea_leaf_ppcg_calc_p_kernel_cuda_(double *beta)
     CHECK_INIT();
     REQUIRE_SOLVER(1 << SOLVER_PPCG);
     BY_PRECISION(ppcg_calc_p_impl, *beta);
+}
+
+// ---- resident runs (no reference counterpart) ----------------------------------------
+//
+// Many iterations in one launch (resident.hpp) for every mesh whose fields fit
+// the chip (about 1500^2 cells in FP64, 2000^2 in FP32): a run wins from the
+// smallest to the largest of them (whole decks: 2.7 times at 10^2 cells, 4.9 at
+// 1000^2; at 1531 x 997, four strips per wave, PPCG 1.7 times).  TEA_RESIDENT=0
+// turns them off, and so does any switch that picks a form of the separate
+// kernels.
+namespace {
+bool resident_tiles(res::Tiles &t)
+{
+    static const char *forms[] = {"TEA_MARCH_CHUNK", "TEA_INNER_RING", "TEA_INNER_MARCH", "TEA_W_FROM_P",
+                                  "TEA_SD_FROM_R", "TEA_FUSED_END", "TEA_END_STORE_R", "TEA_BEGIN_MARCH",
+                                  "TEA_BEGIN_WAVES", "TEA_FUSED_CHEBY", "TEA_CHEBY_PASSES", "TEA_CHEBY_WAVES",
+                                  "TEA_CG_Z_FROM_R", "TEA_FUSED_INNER", "TEA_GRID_MAX", "TEA_SPECULATE",
+                                  "TEA_SPEC_MARGIN", "TEA_PPCG_ITERATION", "TEA_INNER_PASSES"};
+    const char *env = getenv("TEA_RESIDENT");
+    if (g.res_busy || (env && env[0] == '0')) return false;
+    for (const char *f : forms)
+        if (getenv(f)) return false;
+    return res::plan_tiles(t, g.nx, g.ny, g.h, g.fp32 ? g.pitch32 : g.pitch, g.fp32 ? 32 : 64, cu_count());
+}
+
+// The exchange of a launch that uses at most `tags` tags; the words are
+// cleared long before the 32-bit tags could come round.
+res::Exchange resident_exchange(unsigned tags)
+{
+    if (g.res_x.tag > 0x7fffffffu) {
+        (void)hipMemsetAsync(g.res_x.red, 0, (res::EXCHANGE_WORDS - 16) * sizeof(res::word_t), g.stream);
+        g.res_x.tag = 0;
+    }
+    res::Exchange x = g.res_x;
+    g.res_x.tag += tags;
+    return x;
+}
+
+res::Stop resident_stop(const double *s)
+{
+    res::Stop st{};
+    st.error_below = s[0];
+    st.switch_after = s[1] < 1e9 ? (int)s[1] : 1000000000;
+    st.switch_error = s[2];
+    st.reliable = s[3] != 0.0;
+    st.have_q = s[4] != 0.0;
+    st.q_ref = s[5];
+    st.rr_ref = s[6];
+    st.delta = s[7];
+    st.target = s[8];
+    return st;
+}
+
+template <typename T> res::Fields<T> resident_fields()
+{
+    res::Fields<T> f{};
+    f.u = FT<T>(F_U);
+    f.p = FT<T>(F_P);
+    f.r = FT<T>(F_R);
+    f.z = FT<T>(X_Z);
+    f.Kx = FT<T>(X_KX);
+    f.Ky = FT<T>(X_KY);
+    f.rstore = FT<T>(X_RSTORE);
+    f.sd = FT<T>(F_SD);
+    f.rtemp = FT<T>(X_RTEMP);
+    f.utemp = FT<T>(X_UTEMP);
+    f.z_in = f.z;
+    f.u0 = FT<T>(X_U0);
+    f.w = FT<T>(X_W);
+    return f;
+}
+
+// Coefficients k0 .. k0 + n - 1 (n at most RES_HISTORY) in device memory, beta's after alpha's.
+const double *resident_coefs(int k0, int n)
+{
+    if (g.res_coef_at != k0 || g.res_coef_n < n) {
+        for (int k = 0; k < n; k++) {
+            g.h_coef[k] = g.ch_a[k0 + k];
+            g.h_coef[res::RES_HISTORY + k] = g.ch_b[k0 + k];
+        }
+        if (hipMemcpyAsync(g.res_coef, g.h_coef, 2 * res::RES_HISTORY * sizeof(double), hipMemcpyHostToDevice,
+                           g.stream) != hipSuccess)
+            return nullptr;
+        g.res_coef_at = k0;
+        g.res_coef_n = n;
+    }
+    return g.res_coef;
+}
+
+// Launches a run, waits for it and returns its iterations; 0 if it did not
+// start or on an error.
+template <typename L> int resident_run(const char *name, L launch_run)
+{
+    hipError_t err;
+    {
+        Timed timed(name);
+        err = launch_run(g.d_run + 4, (res::Outcome *)g.d_run);
+    }
+    if (err != hipSuccess) { die("launch of %s failed: %s", name, hipGetErrorString(err)); return 0; }
+    err = hipStreamSynchronize(g.stream);
+    if (err != hipSuccess) { die("hipStreamSynchronize failed: %s", hipGetErrorString(err)); return 0; }
+    if (g_profile_table && g.prof.on) g.prof.drain(false);
+    const int n = ((const res::Outcome *)g.h_run)->iterations;
+    if (n == -1) { g.res_busy = true; return 0; }
+    if (n < 0) { die("%s: an exchange among the workgroups timed out", name); return 0; }
+    return n;
+}
+
+template <typename T>
+int cg_run_impl(const res::Tiles &t, int with_p, double beta, double rro, int max_its, const double *stop, double *pw,
+                double *rrn)
+{
+    const int its = max_its < res::RES_HISTORY ? max_its : res::RES_HISTORY;
+    const res::Exchange x = resident_exchange(2 * (unsigned)its + 2);
+    const int n = resident_run(nm<T>("cg_resident"), [&](double *history, res::Outcome *out) {
+        return res::launch_cg<T>(t, g.prec, resident_fields<T>(), x, with_p, beta, rro, resident_stop(stop), its,
+                                 history, out, g.stream);
+    });
+    for (int k = 0; k < n; k++) {
+        pw[k] = g.h_run[4 + 2 * k];
+        rrn[k] = g.h_run[5 + 2 * k];
+    }
+    if (n > 0) g.pending_w = 8 * (int)sizeof(T);   // w = A p of the last iteration, as the fused calls leave it
+    return n;
+}
+
+template <typename T>
+int ppcg_run_impl(const res::Tiles &t, int from_inner, int with_p, double beta, double rro, double theta,
+                  int inner_steps, int max_its, const double *stop, double *values, int *at_ur, double *rrn_end)
+{
+    const int bits = 8 * (int)sizeof(T);
+    const double *coef = resident_coefs(0, inner_steps);
+    if (!coef) { die("tea_engine_ppcg_run: uploading the coefficients failed"); return 0; }
+    // the longest run whose tags fit well inside their range
+    int its = max_its < res::RES_HISTORY ? max_its : res::RES_HISTORY;
+    const unsigned per = (unsigned)inner_steps + 2;
+    const res::Exchange x = resident_exchange(per * ((unsigned)its + 1) + 2);
+    res::Fields<T> f = resident_fields<T>();
+    if (from_inner) {
+        settle_z_utemp();
+        with_p = 0;
+    } else {
+        settle_z_r();
+        // (a run that may end at its first ur keeps z where it has no preconditioner)
+        if (g.pending_z == bits && !(g.prec == PREC_NONE && stop[3] != 0.0)) f.z_in = f.utemp;
+        else settle_z_utemp();
+    }
+    const int n = resident_run(nm<T>("ppcg_resident"), [&](double *history, res::Outcome *out) {
+        return res::launch_ppcg<T>(t, g.prec, f, x, from_inner, with_p, beta, rro, theta, coef, res::RES_HISTORY,
+                                   inner_steps, resident_stop(stop), its, history, out, g.stream);
+    });
+    if (n < 1) return n;
+    const res::Outcome *o = (const res::Outcome *)g.h_run;
+    for (int k = 0; k < 4 * n; k++) values[k] = g.h_run[4 + k];
+    *at_ur = o->at_ur;
+    *rrn_end = o->rrn_end;
+    if (o->at_ur) values[4 * n - 1] = 0.0;
+    g.pending_w = bits;                       // w = A p, as the fused calls leave it
+    g.pending_zr = g.pending_sd_r = 0;
+    g.pending_rt_ut = o->at_ur ? bits : 0;    // rtemp = r, utemp = sd
+    g.pending_z = o->at_ur ? 0 : bits;        // z = utemp
+    return n;
+}
+
+template <typename T>
+int cheby_run_impl(const res::Tiles &t, int k0, int n0, int check_from, double error, double target, int max_its,
+                   double *rr)
+{
+    const int its = max_its < res::RES_HISTORY ? max_its : res::RES_HISTORY;
+    const double *coef = resident_coefs(k0, its);
+    if (!coef) { die("tea_engine_cheby_run: uploading the coefficients failed"); return 0; }
+    const res::Exchange x = resident_exchange((unsigned)its + 2);
+    const int n = resident_run(nm<T>("cheby_resident"), [&](double *history, res::Outcome *out) {
+        return res::launch_cheby<T>(t, g.prec, resident_fields<T>(), x, coef, res::RES_HISTORY, n0, check_from, error,
+                                    target, its, history, out, g.stream);
+    });
+    for (int k = 0; k < n; k++) rr[k] = g.h_run[4 + k];
+    return n;
+}
+}  // namespace
+
+#define RUN_CHECK(mask)                                                                                   \
+    do {                                                                                                  \
+        if (!g.initialised) { die("%s called before initialise_cuda_", __func__); return 0; }             \
+        if (!((mask) & (1 << g.solver))) {                                                                \
+            die("%s: kernel not registered for the solver selected in the deck", __func__);               \
+            return 0;                                                                                     \
+        }                                                                                                 \
+    } while (0)
+
+EXPORT int tea_engine_cg_run(int with_p, double beta, double rro, int max_its, const double *stop, double *pw,
+                             double *rrn)
+{
+    RUN_CHECK(S_CG_FAMILY);
+    res::Tiles t;
+    if (max_its < 1 || !resident_tiles(t)) return 0;
+    g.calls++;
+    g.pending_w = 0;   // rewritten
+    settle_pending();
+    return BY_PRECISION(cg_run_impl, t, with_p, beta, rro, max_its, stop, pw, rrn);
+}
+
+EXPORT int tea_engine_ppcg_run(int from_inner, int with_p, double beta, double rro, double theta, int inner_steps,
+                               int max_its, const double *stop, double *values, int *at_ur, double *rrn_end)
+{
+    RUN_CHECK(1 << SOLVER_PPCG);
+    if (inner_steps < 0 || inner_steps > (int)g.ch_a.size()) {
+        die("ppcg_run: %d inner steps, %d coefficients uploaded", inner_steps, (int)g.ch_a.size());
+        return 0;
+    }
+    res::Tiles t;
+    if (max_its < 1 || inner_steps > res::RES_HISTORY || !resident_tiles(t)) return 0;
+    g.calls++;
+    if (!from_inner) drop_w_settle_rest();
+    return BY_PRECISION(ppcg_run_impl, t, from_inner, with_p, beta, rro, theta, inner_steps, max_its, stop, values,
+                        at_ur, rrn_end);
+}
+
+EXPORT int tea_engine_cheby_run(int step, int n, int check_from, double error, double target, int max_its, double *rr)
+{
+    RUN_CHECK(1 << SOLVER_CHEBY);
+    const int k = step - 1;
+    if (k < 0 || max_its < 1 || k + max_its > (int)g.ch_a.size()) {
+        die("cheby_run: steps %d..%d outside the %d uploaded coefficients", step, step + max_its - 1,
+            (int)g.ch_a.size());
+        return 0;
+    }
+    res::Tiles t;
+    if (!resident_tiles(t)) return 0;
+    g.calls++;
+    g.pending_cheby = 0;   // the iterations form w and r again
+    settle_pending();
+    return BY_PRECISION(cheby_run_impl, t, k, n, check_from, error, target, max_its, rr);
 }
 
 // =============================================================================

@@ -106,47 +106,6 @@ __device__ __forceinline__ void block_reduce(DD (&v)[NV], const Red red)
     }
 }
 
-// Combines the nblocks partials of each of nv values (lane t takes partials
-// t, t+1024, ...; then the wave and workgroup trees) and writes out[j] =
-// rounded sum.  Launched with one workgroup of FINISH_THREADS threads.
-constexpr int FINISH_THREADS = 1024;
-
-__global__ __launch_bounds__(FINISH_THREADS) void k_finish(const DD *__restrict__ partials, int max_blocks,
-                                                          int nblocks, int nv, double *__restrict__ out,
-                                                          double *__restrict__ dev_out)
-{
-    __shared__ DD lds[FINISH_THREADS / WAVE];
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int wave = threadIdx.x / WAVE;
-    for (int j = 0; j < nv; j++) {
-        DD acc{0.0, 0.0};
-        const DD *p = partials + (size_t)j * max_blocks;
-        // lane t merges partials t, t+1024, ... in that order; eight loads are
-        // issued before the first merge waits
-        for (int b0 = threadIdx.x; b0 < nblocks; b0 += 8 * FINISH_THREADS) {
-            DD x[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int b = b0 + u * FINISH_THREADS;
-                x[u] = b < nblocks ? p[b] : DD{0.0, 0.0};
-            }
-#pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (b0 + u * FINISH_THREADS < nblocks) dd_merge(acc, x[u]);
-        }
-        acc = wave_reduce(acc);
-        if (lane == 0) lds[wave] = acc;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            DD t = lds[0];
-            for (int w = 1; w < FINISH_THREADS / WAVE; w++) dd_merge(t, lds[w]);
-            out[j] = t.s + t.c;
-            if (dev_out) dev_out[j] = t.s + t.c;   // for a following launch on the device
-        }
-        __syncthreads();
-    }
-}
-
 // Column and first row of a lane's strip; len = rows in the strip (0 if none).
 struct Strip {
     int c, r0, len;

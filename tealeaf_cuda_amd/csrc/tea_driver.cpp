@@ -101,6 +101,9 @@ struct Backend {
     void (*cheby_iterate_n)(int, int) = nullptr;
     int (*ppcg_inner_plan)(int) = nullptr;
     void (*cg_begin_ur)(int, double, double, double *, double *) = nullptr;
+    int (*cg_run)(int, double, double, int, const double *, double *, double *) = nullptr;
+    int (*ppcg_run)(int, int, double, double, double, int, int, const double *, double *, int *, double *) = nullptr;
+    int (*cheby_run)(int, int, int, double, double, int, double *) = nullptr;
 
     void check() const
     {
@@ -151,6 +154,13 @@ Backend load_backend(const char *path)
     b.cheby_iterate_n = reinterpret_cast<void (*)(int, int)>(dlsym(b.handle, "tea_engine_cheby_iterate_n"));
     b.cg_begin_ur =
         reinterpret_cast<void (*)(int, double, double, double *, double *)>(dlsym(b.handle, "tea_engine_cg_begin_ur"));
+    b.cg_run = reinterpret_cast<int (*)(int, double, double, int, const double *, double *, double *)>(
+        dlsym(b.handle, "tea_engine_cg_run"));
+    b.ppcg_run =
+        reinterpret_cast<int (*)(int, int, double, double, double, int, int, const double *, double *, int *, double *)>(
+            dlsym(b.handle, "tea_engine_ppcg_run"));
+    b.cheby_run = reinterpret_cast<int (*)(int, int, int, double, double, int, double *)>(
+        dlsym(b.handle, "tea_engine_cheby_run"));
     return b;
 }
 
@@ -593,6 +603,8 @@ private:
     } rel;
     bool reliable_step(double q, bool refresh_z, bool *replaced);
     bool replacement_unlikely() const;
+    bool replacement_due(double q) const;
+    void run_stop(double *stop, double error_below) const;
     void run_ppcg_inner_steps(int *ppcg_inner_iters, bool fused = false);
     // the fused outer iteration (tea_engine_ppcg_begin/ur/end) is used when the
     // backend has it and no halo update separates the fused calls
@@ -968,11 +980,63 @@ Run::Solve Run::iterate(double initial_residual_sq, double eps)
 
     // fused CG iterations (tea_engine_cg_begin_ur): the calc_p of each
     // iteration is applied by the next call, or by the separate entry point
-    // when the CG branch is left (not under residual replacement, whose
-    // updates fall between calc_ur and calc_p's successor)
+    // when the CG branch is left or a residual replacement follows (which
+    // comes after calc_p)
     const char *fused_cg_env = std::getenv("TEA_FUSED_CG");
-    const bool fused_cg = cg_family && b.cg_begin_ur && !d.reflective_boundary && !rel.on &&
+    const bool fused_cg = cg_family && b.cg_begin_ur && !d.reflective_boundary &&
                           !(fused_cg_env && fused_cg_env[0] == '0');
+    // runs of them in one call (tea_engine_cg_run): the values of the
+    // iterations run ahead wait here until the loop reaches them
+    bool cg_runs = fused_cg && b.cg_run;
+    std::vector<double> run_pw, run_rrn;
+    size_t run_next = 0;
+    // Chebyshev iterations likewise (tea_engine_cheby_run)
+    bool cheby_runs = cheby_batch && b.cheby_run;
+    // and whole outer iterations of PPCG (tea_engine_ppcg_run): four values of each
+    const char *runs_env = std::getenv("TEA_RESIDENT");
+    bool ppcg_runs = fused && b.ppcg_run && b.ppcg_inner_n && b.ppcg_inner_plan && d.tl_ppcg_inner_steps > 0 &&
+                     !(rel.on && d.verbose_on) && !(passes_env && passes_env[0] == '0') &&
+                     !(runs_env && runs_env[0] == '0');
+    std::vector<double> outer;
+    size_t outer_next = 0;
+    int outer_at_ur = 0;
+    bool inner_due = false;       // the latest iteration still lacks its inner steps and end
+    double outer_end = 0.0;
+    // the inner steps and the end it lacks, by the separate calls
+    auto finish_outer = [&](bool form_sd) {
+        if (form_sd) {
+            double th = theta;
+            b.tea_leaf_ppcg_init_sd_new_kernel_cuda_(&th);
+            b.check();
+        }
+        run_ppcg_inner_steps(&ppcg_inner_iters, true);
+        b.ppcg_end(&outer_end);
+        b.check();
+        inner_due = false;
+        p_pending = true;
+        beta_pending = outer_end / rro_begin;
+    };
+    // Makes the next outer iteration's values available; false where runs do not apply.
+    auto next_outer = [&]() -> bool {
+        if (!ppcg_runs) return false;
+        if (outer_next < outer.size()) return true;
+        double stop[9];
+        run_stop(stop, eps * initial_residual);
+        const int room = std::min(max_iters - n + 1, 1024);
+        outer.resize(4 * (size_t)room);
+        const int done = b.ppcg_run(inner_due ? 1 : 0, !inner_due && p_pending ? 1 : 0, beta_pending, rro_begin, theta,
+                                    d.tl_ppcg_inner_steps, room, stop, outer.data(), &outer_at_ur, &outer_end);
+        b.check();
+        outer.resize(4 * (size_t)done);
+        outer_next = 0;
+        if (done == 0) {   // the mesh does not fit
+            ppcg_runs = false;
+            if (inner_due) finish_outer(rel.bits != 32 || !b.mp_replace);
+            return false;
+        }
+        inner_due = false;
+        return true;
+    };
     bool cg_p_pending = false;
     double cg_beta_pending = 0.0;
     auto flush_cg_p = [&]() {
@@ -982,6 +1046,20 @@ Run::Solve Run::iterate(double initial_residual_sq, double eps)
         cg_p_pending = false;
     };
 
+    // Makes the next Chebyshev iteration's value available (run_rrn), likewise.
+    auto next_cheby = [&]() -> bool {
+        if (run_next < run_rrn.size()) return true;
+        const int room = std::min(std::min(max_iters - n + 1, 1024), max_cheby_iters - cheby_calc_steps + 1);
+        run_rrn.resize(std::max(room, 0));
+        run_next = 0;
+        const int done = room < 1 ? 0 : b.cheby_run(cheby_calc_steps, n, est_itc, error, eps * initial_residual, room,
+                                                    run_rrn.data());
+        b.check();
+        run_rrn.resize(done);
+        if (done == 0) cheby_runs = false;
+        return done > 0;
+    };
+
     for (n = 1; n <= max_iters; n++) {
         if (!ch_switch_check) {
             if (cheby_calc_steps > 0) ch_switch_check = true;
@@ -989,7 +1067,10 @@ Run::Solve Run::iterate(double initial_residual_sq, double eps)
             else if (std::fabs(old_error) <= d.tl_ch_cg_epslim && n >= d.tl_ch_cg_presteps) ch_switch_check = true;
             else ch_switch_check = false;
         }
-        if ((d.tl_use_chebyshev || d.tl_use_ppcg) && ch_switch_check) flush_cg_p();
+        if ((d.tl_use_chebyshev || d.tl_use_ppcg) && ch_switch_check) {
+            if (run_next < run_rrn.size() && cheby_calc_steps == 0) fail("a run of CG iterations went past the switch");
+            flush_cg_p();
+        }
 
         if ((d.tl_use_chebyshev || d.tl_use_ppcg) && ch_switch_check) {
             if (cheby_calc_steps == 0) {
@@ -1054,6 +1135,9 @@ Run::Solve Run::iterate(double initial_residual_sq, double eps)
                     est_itc = (int)std::lround(std::log(it_alpha) / (2.0 * std::log(gamm)));
                     log("    est itc\n%11d\n", est_itc);
                     cheby_calc_steps = 1;
+                } else if (cheby_runs && next_cheby()) {
+                    if (n >= est_itc && n % 10 == 0) error = run_rrn[run_next];
+                    run_next++;
                 } else if (cheby_batch) {
                     // iterations n .. last in streaming passes: up to the next
                     // norm check, tl_max_iters, the last coefficient, or the
@@ -1093,6 +1177,31 @@ Run::Solve Run::iterate(double initial_residual_sq, double eps)
                         b.check();
                     }
                 }
+            } else if (d.tl_use_ppcg && next_outer()) {
+                // the calls of the branches below, made ahead
+                const double *v = &outer[outer_next];
+                outer_next += 4;
+                const bool last = outer_next == outer.size();
+                pw = v[0];
+                rro = v[1];
+                rro_begin = rro;
+                if (rel.on) {
+                    rrn = v[2];
+                    bool replaced = false;
+                    const int updates_before = rel.updates;
+                    if (reliable_step(rrn, true, &replaced)) converged = true;
+                    else ppcg_inner_iters += d.tl_ppcg_inner_steps;
+                    if ((converged || rel.updates != updates_before) && !(last && outer_at_ur))
+                        fail("a run of outer iterations went past a residual replacement");
+                } else {
+                    rrn = v[3];
+                    ppcg_inner_iters += d.tl_ppcg_inner_steps;
+                }
+                inner_due = last && outer_at_ur && !converged;
+                p_pending = !inner_due;
+                beta_pending = v[3] / rro;
+                error = rrn;
+                rro = rrn;
             } else if (d.tl_use_ppcg && whole_iteration) {
                 // the calls of the branch below in one: begin_ur, the inner
                 // steps, end (rrn)
@@ -1195,14 +1304,47 @@ Run::Solve Run::iterate(double initial_residual_sq, double eps)
         } else if (cg_family && fused_cg) {
             // the calls below in one: [calc_p(beta) of the previous iteration], calc_w, calc_ur
             fields[FIELD_P - 1] = 1;
-            b.cg_begin_ur(cg_p_pending ? 1 : 0, cg_beta_pending, rro, &pw, &rrn);
-            b.check();
+            if (cg_runs && run_next == run_rrn.size()) {
+                // iterations up to the loop's next decision: the switch to
+                // Chebyshev or PPCG (tested at the top of the loop), its stop,
+                // a residual replacement, tl_max_iters
+                double stop[9];
+                run_stop(stop, eps * initial_residual);
+                int room = std::min(max_iters - n + 1, 1024);
+                if (d.tl_use_chebyshev || d.tl_use_ppcg) {
+                    if (!first && d.tl_use_ppcg) room = 1;
+                    stop[1] = std::max(1, d.tl_ch_cg_presteps - n);
+                    stop[2] = d.tl_ch_cg_epslim;
+                }
+                run_pw.resize(room);
+                run_rrn.resize(room);
+                const int done = room > 1 ? b.cg_run(cg_p_pending ? 1 : 0, cg_beta_pending, rro, room, stop,
+                                                     run_pw.data(), run_rrn.data()) : 0;
+                b.check();
+                run_pw.resize(done);
+                run_rrn.resize(done);
+                run_next = 0;
+                if (room > 1 && done == 0) cg_runs = false;   // the mesh does not fit
+            }
+            if (run_next < run_rrn.size()) {
+                pw = run_pw[run_next];
+                rrn = run_rrn[run_next];
+                run_next++;
+            } else {
+                b.cg_begin_ur(cg_p_pending ? 1 : 0, cg_beta_pending, rro, &pw, &rrn);
+                b.check();
+            }
             alpha = rro / pw;
             cg_alphas[n] = alpha;
             beta = rrn / rro;
             cg_betas[n] = beta;
-            cg_p_pending = true;
+            cg_p_pending = run_next == run_rrn.size();   // else applied inside the run
             cg_beta_pending = beta;
+            if (rel.on) {
+                if (replacement_due(rrn)) flush_cg_p();   // calc_p comes first
+                // a replaced r reaches z at the next cg_calc_ur
+                if (reliable_step(rrn, false, nullptr)) converged = true;
+            }
             error = rrn;
             rro = rrn;
         } else if (cg_family) {
@@ -1227,16 +1369,29 @@ Run::Solve Run::iterate(double initial_residual_sq, double eps)
         }
 
         update_halo(fields, 1);
-        if (converged) break;
+        const bool ahead = run_next < run_rrn.size() || outer_next < outer.size();
+        if (converged) {
+            if (ahead) fail("a run of iterations went past the solve's end");
+            break;
+        }
 
         error = std::sqrt(std::fabs(error));
         if (d.verbose_on) log(" Residual %.16E\n", error);
-        if (std::fabs(error) < eps * initial_residual) break;
+        if (std::fabs(error) < eps * initial_residual) {
+            if (ahead) fail("a run of iterations went past the solve's end");
+            break;
+        }
         old_error = error;
     }
     flush_cg_p();
     // a DO loop that runs to completion leaves n = max_iters + 1
-    if (end_pending) {   // stopped by tl_max_iters: complete the last outer iteration
+    if (inner_due) {     // stopped by tl_max_iters: complete the last outer iteration
+        finish_outer(rel.bits != 32 || !b.mp_replace);
+        error = std::sqrt(std::fabs(outer_end));
+    } else if (rel.on && !converged && !outer.empty()) {
+        error = std::sqrt(std::fabs(outer_end));
+    }
+    if (end_pending) {   // the same
         b.ppcg_end(&rrn);
         b.check();
         error = std::sqrt(std::fabs(rrn));
@@ -1395,6 +1550,24 @@ bool Run::replacement_unlikely() const
     const double drop = std::sqrt(q_next / std::fabs(rel.q_ref));
     const double predicted = std::sqrt(std::fabs(rel.rr_ref)) * drop;
     return drop >= margin * d.reliable_delta && predicted >= margin * rel.target;
+}
+
+// Whether reliable_step(q) will replace the residual (or end the solve).
+bool Run::replacement_due(double q) const
+{
+    if (!rel.have_q) return false;
+    const double drop = std::sqrt(std::fabs(q / rel.q_ref));
+    const double predicted = std::sqrt(std::fabs(rel.rr_ref)) * drop;
+    return !(drop >= d.reliable_delta && predicted >= rel.target);
+}
+
+// The tests that end a run of iterations (include/tea_leaf_engine.h): the
+// loop's own stop and, under residual replacement, replacement_due.
+void Run::run_stop(double *stop, double error_below) const
+{
+    const double s[9] = {error_below, (double)d.max_iters + 1.0, -1.0, rel.on ? 1.0 : 0.0, rel.have_q ? 1.0 : 0.0,
+                         rel.q_ref, rel.rr_ref, d.reliable_delta, rel.target};
+    std::copy(s, s + 9, stop);
 }
 
 bool Run::reliable_step(double q, bool refresh_z, bool *replaced)

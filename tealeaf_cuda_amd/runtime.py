@@ -124,6 +124,14 @@ _EXT = {
     "tea_engine_ppcg_inner_plan": ([ctypes.c_int], ctypes.c_int),
     "tea_engine_cg_begin_ur": ([ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.POINTER(ctypes.c_double),
                                 ctypes.POINTER(ctypes.c_double)], None),
+    "tea_engine_cg_run": ([ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_int,
+                           ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double),
+                           ctypes.POINTER(ctypes.c_double)], ctypes.c_int),
+    "tea_engine_ppcg_run": ([ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+                             ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_double),
+                             ctypes.POINTER(ctypes.c_double), _I, ctypes.POINTER(ctypes.c_double)], ctypes.c_int),
+    "tea_engine_cheby_run": ([ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_double, ctypes.c_double,
+                              ctypes.c_int, ctypes.POINTER(ctypes.c_double)], ctypes.c_int),
     "tea_engine_set_precision": ([ctypes.c_int], ctypes.c_int),
     "tea_engine_mp_leave": ([], ctypes.c_int),
     "tea_engine_mp_setup": ([], None),
@@ -415,6 +423,31 @@ class Engine:
         self._call("tea_engine_cg_begin_ur", int(bool(with_p)), float(beta), float(rro), ctypes.byref(pw),
                    ctypes.byref(rrn))
         return pw.value, rrn.value
+
+    def cg_run(self, with_p: bool, beta: float, rro: float, max_its: int, stop):
+        """Returns the lists pw, rrn of the calls made (empty: the mesh does not fit)."""
+        pw, rrn = (ctypes.c_double * max_its)(), (ctypes.c_double * max_its)()
+        n = self.lib.tea_engine_cg_run(int(bool(with_p)), float(beta), float(rro), int(max_its), _darr(stop), pw, rrn)
+        self._check()
+        return list(pw[:n]), list(rrn[:n])
+
+    def ppcg_run(self, from_inner: bool, with_p: bool, beta: float, rro: float, theta: float, inner_steps: int,
+                 max_its: int, stop):
+        """Returns (values: a list of (pw, rz, rrn_ur, rrn_end) per iteration, at_ur, rrn_end)."""
+        v, at_ur, end = (ctypes.c_double * (4 * max_its))(), ctypes.c_int(), ctypes.c_double()
+        n = self.lib.tea_engine_ppcg_run(int(bool(from_inner)), int(bool(with_p)), float(beta), float(rro),
+                                         float(theta), int(inner_steps), int(max_its), _darr(stop), v,
+                                         ctypes.byref(at_ur), ctypes.byref(end))
+        self._check()
+        return [tuple(v[4 * k:4 * k + 4]) for k in range(n)], bool(at_ur.value), end.value
+
+    def cheby_run(self, step: int, n: int, check_from: int, error: float, target: float, max_its: int):
+        """Returns the r.r of each iteration made (0 where it is not formed)."""
+        rr = (ctypes.c_double * max_its)()
+        k = self.lib.tea_engine_cheby_run(int(step), int(n), int(check_from), float(error), float(target),
+                                          int(max_its), rr)
+        self._check()
+        return list(rr[:k])
 
     def ppcg_end(self) -> float:
         out = ctypes.c_double()
