@@ -807,7 +807,7 @@ __device__ __forceinline__ void block_reduce_lanes(const double (&v)[NV], const 
 #pragma unroll
     for (int j = 0; j < NV; j++) {
         const DD t = wave_reduce(DD{v[j], 0.0});
-        if (lane == 0) lds[j][wave] = t;
+        if (lane == WAVE - 1) lds[j][wave] = t;
     }
     __syncthreads();
     if (threadIdx.x == 0) {

@@ -60,15 +60,32 @@ __device__ __forceinline__ void dd_merge(DD &a, const DD b)
     a.c += (se + b.c);
 }
 
+// Lane moves of a double-double by DPP (lanes without a source receive 0, the
+// neutral element of dd_merge).
+template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_double(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ void dpp_merge(DD &v)
+{
+    DD o;
+    o.s = dpp_double<CTRL, ROWS>(v.s);
+    o.c = dpp_double<CTRL, ROWS>(v.c);
+    dd_merge(v, o);
+}
+// Sum over the wave, in its last lane (row shifts by 1, 2, 4, 8, then the row
+// broadcasts): register moves, where shuffles go through LDS.
 __device__ __forceinline__ DD wave_reduce(DD v)
 {
-#pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) {
-        DD o;
-        o.s = __shfl_xor(v.s, off, WAVE);
-        o.c = __shfl_xor(v.c, off, WAVE);
-        dd_merge(v, o);
-    }
+    dpp_merge<0x111, 0xf>(v);
+    dpp_merge<0x112, 0xf>(v);
+    dpp_merge<0x114, 0xf>(v);
+    dpp_merge<0x118, 0xf>(v);
+    dpp_merge<0x142, 0xa>(v);
+    dpp_merge<0x143, 0xc>(v);
     return v;
 }
 
@@ -91,7 +108,7 @@ __device__ __forceinline__ void block_reduce(DD (&v)[NV], const Red red)
     const int wave = threadIdx.x / WAVE;
 #pragma unroll
     for (int j = 0; j < NV; j++) v[j] = wave_reduce(v[j]);
-    if (lane == 0) {
+    if (lane == WAVE - 1) {
 #pragma unroll
         for (int j = 0; j < NV; j++) lds[j][wave] = v[j];
     }

@@ -14,23 +14,27 @@
 
 namespace tea {
 
-// Combines the nblocks partials of each of nv values (lane t takes partials
-// t, t+1024, ...; then the wave and workgroup trees) and writes out[j] =
-// rounded sum.  Launched with one workgroup of FINISH_THREADS threads.
+// Combines the nblocks partials of each of nv values (thread t takes partials
+// t, t+1024, ...; then the wave trees) and writes out[j] = rounded sum.
+// Launched with one workgroup of FINISH_THREADS threads.  A serial chain of
+// FP64 merges: each wave sums whole values' wave sums by a tree, after one
+// barrier (with one value after the other, sixteen wave sums merged in turn and
+// shuffles through LDS, a CG iteration with its two reductions took 35.2 us at
+// 250^2 cells, now 33.0; 339.3 and 337.4 at 4000^2).
 constexpr int FINISH_THREADS = 1024;
 
 __global__ __launch_bounds__(FINISH_THREADS) void k_finish(const DD *__restrict__ partials, int max_blocks,
                                                           int nblocks, int nv, double *__restrict__ out,
                                                           double *__restrict__ dev_out)
 {
-    __shared__ DD lds[FINISH_THREADS / WAVE];
+    constexpr int NW = FINISH_THREADS / WAVE;
+    __shared__ DD lds[MAX_RED][NW];
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = threadIdx.x / WAVE;
     for (int j = 0; j < nv; j++) {
         DD acc{0.0, 0.0};
         const DD *p = partials + (size_t)j * max_blocks;
-        // lane t merges partials t, t+1024, ... in that order; eight loads are
-        // issued before the first merge waits
+        // eight loads are issued before the first merge waits
         for (int b0 = threadIdx.x; b0 < nblocks; b0 += 8 * FINISH_THREADS) {
             DD x[8];
 #pragma unroll
@@ -43,15 +47,15 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_finish(const DD *__restrict_
                 if (b0 + u * FINISH_THREADS < nblocks) dd_merge(acc, x[u]);
         }
         acc = wave_reduce(acc);
-        if (lane == 0) lds[wave] = acc;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            DD t = lds[0];
-            for (int w = 1; w < FINISH_THREADS / WAVE; w++) dd_merge(t, lds[w]);
+        if (lane == WAVE - 1) lds[j][wave] = acc;
+    }
+    __syncthreads();
+    for (int j = wave; j < nv; j += NW) {
+        const DD t = wave_reduce(lane < NW ? lds[j][lane] : DD{0.0, 0.0});
+        if (lane == WAVE - 1) {
             out[j] = t.s + t.c;
             if (dev_out) dev_out[j] = t.s + t.c;   // for a following launch on the device
         }
-        __syncthreads();
     }
 }
 

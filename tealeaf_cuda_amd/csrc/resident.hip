@@ -31,34 +31,6 @@ __device__ __forceinline__ void store_word(word_t *p, unsigned tag, unsigned dat
     __hip_atomic_store(p, ((word_t)tag << 32) | data, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Lane moves of a double-double by DPP (lanes without a source receive 0, the
-// neutral element of dd_merge).
-template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_double(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-template <int CTRL, int ROWS> __device__ __forceinline__ void dpp_merge(DD &v)
-{
-    DD o;
-    o.s = dpp_double<CTRL, ROWS>(v.s);
-    o.c = dpp_double<CTRL, ROWS>(v.c);
-    dd_merge(v, o);
-}
-// Sum over the wave in lane 63 (row shifts by 1, 2, 4, 8, then the row
-// broadcasts): register moves where shuffles go through LDS.
-__device__ __forceinline__ DD wave_sum63(DD v)
-{
-    dpp_merge<0x111, 0xf>(v);
-    dpp_merge<0x112, 0xf>(v);
-    dpp_merge<0x114, 0xf>(v);
-    dpp_merge<0x118, 0xf>(v);
-    dpp_merge<0x142, 0xa>(v);
-    dpp_merge<0x143, 0xc>(v);
-    return v;
-}
 __device__ __forceinline__ double lane_value(double v, int lane)
 {
     const long long b = __double_as_longlong(v);
@@ -266,7 +238,7 @@ template <typename T, int S> struct Place {
     {
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-            const DD t = wave_sum63(acc[v]);
+            const DD t = wave_reduce(acc[v]);
             if (lane == WAVE - 1) sh.part[v][wave] = t;
         }
     }
@@ -312,7 +284,7 @@ template <typename T, int S> struct Place {
             DD t;
             t.s = __longlong_as_double((long long)((q[0] & 0xffffffffull) | (q[1] << 32)));
             t.c = __longlong_as_double((long long)((q[2] & 0xffffffffull) | (q[3] << 32)));
-            t = wave_sum63(t);
+            t = wave_reduce(t);
             if (lane == WAVE - 1) sh.sum[v][wave] = t;
         }
     }
