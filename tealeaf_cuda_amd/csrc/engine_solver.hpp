@@ -20,12 +20,15 @@ namespace tea {
 // FP64 merges: each wave sums whole values' wave sums by a tree, after one
 // barrier (with one value after the other, sixteen wave sums merged in turn and
 // shuffles through LDS, a CG iteration with its two reductions took 35.2 us at
-// 250^2 cells, now 33.0; 339.3 and 337.4 at 4000^2).
+// 250^2 cells, now 33.0; 339.3 and 337.4 at 4000^2).  words (if given; host memory): value j in two words of 32 bits each
+// with `tag` above them, so the host sees when a value is whole without waiting
+// for the launch to be retired.
 constexpr int FINISH_THREADS = 1024;
 
 __global__ __launch_bounds__(FINISH_THREADS) void k_finish(const DD *__restrict__ partials, int max_blocks,
                                                           int nblocks, int nv, double *__restrict__ out,
-                                                          double *__restrict__ dev_out)
+                                                          double *__restrict__ dev_out,
+                                                          unsigned long long *__restrict__ words, unsigned tag)
 {
     constexpr int NW = FINISH_THREADS / WAVE;
     __shared__ DD lds[MAX_RED][NW];
@@ -53,8 +56,17 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_finish(const DD *__restrict_
     for (int j = wave; j < nv; j += NW) {
         const DD t = wave_reduce(lane < NW ? lds[j][lane] : DD{0.0, 0.0});
         if (lane == WAVE - 1) {
-            out[j] = t.s + t.c;
-            if (dev_out) dev_out[j] = t.s + t.c;   // for a following launch on the device
+            const double sum = t.s + t.c;
+            if (out) out[j] = sum;
+            if (dev_out) dev_out[j] = sum;   // for a following launch on the device
+            if (words) {
+                const unsigned long long b = (unsigned long long)__double_as_longlong(sum);
+                const unsigned long long above = (unsigned long long)tag << 32;
+                __hip_atomic_store(words + 2 * j, above | (b & 0xffffffffull), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_SYSTEM);
+                __hip_atomic_store(words + 2 * j + 1, above | (b >> 32), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_SYSTEM);
+            }
         }
     }
 }
