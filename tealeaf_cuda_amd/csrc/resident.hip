@@ -76,7 +76,7 @@ template <int S, typename T, int N> __device__ __forceinline__ T get_last(const 
 template <typename T, int S> struct Shared {
     static constexpr int R = S * STRIP;
     static constexpr int NW = R * (int)sizeof(T) / 4;   // 32-bit words of a column face per wave
-    static_assert(NW <= WAVE, "one word per lane and side");
+    static_assert(NW <= FACE_WORDS, "a lane per word");
     unsigned face[RES_WAVES][2][NW];    // column faces on their way out and in
     T rows[2][RES_WAVES][2][WAVE];      // [slot] first and last row of each wave
     DD part[2][RES_WAVES];
@@ -145,6 +145,18 @@ template <typename T, int S> struct Place {
     }
 
     __device__ int strip_len(int k) const { return max(0, min(STRIP, nrows - k * STRIP)); }
+    // Sets what strip k has beyond its rows to 0 (a test per strip: only a
+    // tile's last one, at the top of the mesh, is ever short).
+    template <int N> __device__ void cut(int k, T (&v)[N], int at = 0) const
+    {
+        if ((k + 1) * STRIP <= nrows) return;
+        asm volatile("" ::: "memory");   // a branch, not selects on every row
+#pragma unroll
+        for (int i = 0; i < STRIP; i++)
+            if (k * STRIP + i >= nrows) v[at + i] = T(0.0);
+    }
+    // acc without the lanes that own no column
+    __device__ DD owned(DD acc) const { return DD{out ? acc.s : 0.0, out ? acc.c : 0.0}; }
     // row r0 + j (j < n) at lane offset o
     __device__ T load(const FieldBuf<T> &b, unsigned o, int j, int n) const
     {
@@ -376,7 +388,7 @@ private:
     }
     __device__ word_t *col_at(int slot, int w, int side) const
     {
-        return x.col + (((size_t)(slot * RES_MAX_WG + w) * 2 + side) * RES_WAVES + wave) * WAVE + lane;
+        return x.col + (((size_t)(slot * RES_MAX_WG + w) * 2 + side) * RES_WAVES + wave) * FACE_WORDS + lane;
     }
     __device__ word_t *row_at(int slot, int w, int side) const
     {
@@ -639,14 +651,16 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_cg_resident(Tiles t, Fields<T>
         for (int k = 0; k < S; k++) {
             if (k < w.mine) {
 #pragma unroll
+                for (int i = 0; i < STRIP; i++) v[k * STRIP + i] = co.apply(w, p, pb, k * STRIP + i);
+                w.cut(k, v, k * STRIP);
+#pragma unroll
                 for (int i = 0; i < STRIP; i++) {
                     const int j = k * STRIP + i;
-                    const T a = co.apply(w, p, pb, j);
-                    v[j] = w.out && j < w.nrows ? a : T(0.0);
                     dd_add_prod(acc[0], (double)p[j], (double)v[j]);
                 }
             }
         }
+        acc[0] = w.owned(acc[0]);
         w.template part<1>(sh, acc);
         __syncthreads();
         w.template post_total<1>(sh);
@@ -667,14 +681,15 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_cg_resident(Tiles t, Fields<T>
                     rv[i] = r[j];
                 }
                 fac.apply(w, co, k, rv, zv);
+                w.cut(k, zv);
 #pragma unroll
                 for (int i = 0; i < STRIP; i++) {
-                    const int j = k * STRIP + i;
-                    v[j] = w.out && j < w.nrows ? zv[i] : T(0.0);
-                    dd_add_prod(acc[0], (double)rv[i], (double)v[j]);
+                    v[k * STRIP + i] = zv[i];
+                    dd_add_prod(acc[0], (double)rv[i], (double)zv[i]);
                 }
             }
         }
+        acc[0] = w.owned(acc[0]);
         w.post(sh, v);
         w.template part<1>(sh, acc);
         __syncthreads();
@@ -718,8 +733,9 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_cg_resident(Tiles t, Fields<T>
 #pragma unroll
                     for (int i = 0; i < STRIP; i++) {
                         const int j = k * STRIP + i;
-                        if (j < w.nrows) p[j] = v[j] + beta * p[j];
+                        p[j] = v[j] + beta * p[j];
                     }
+                    w.cut(k, p, k * STRIP);
                 }
             }
             if (w.in_above) set_top<S>(p, w.mine, pt);
@@ -750,7 +766,9 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_cg_resident(Tiles t, Fields<T>
 // all-reduce): bound by its latency on small meshes, by issue on the largest.
 // Measured, FP64, a deck's whole run with its CG steps and set-up, against the
 // separate passes: 512^2 block Jacobi, 10 inner steps 4.14 (9.48) ms; 1531 x
-// 997 jac_diag, halo depth 2, to the FP64 true residual 9.89 (17.21) ms.
+// 997 jac_diag, halo depth 2, to the FP64 true residual 9.14 (17.21) ms.  At
+// four strips per wave an inner step takes 6.6 us: 4.7 of issue (with selects
+// per row instead of branches per strip, 5.2), 0.8 before the exchange is in.
 template <typename T, int PREC, int S>
 __global__ __launch_bounds__(RES_BLOCK, 2) void k_ppcg_resident(Tiles t, Fields<T> f, Exchange x, int from_inner,
                                                                 int with_p, double beta_in, double rro,
@@ -954,10 +972,14 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_ppcg_resident(Tiles t, Fields<
                 utb += sdb;
                 set_top<S>(ut, w.mine, get_top<S>(ut, w.mine) + sdt);
             }
-            if (halo_lane) {
+            if (halo_lane && s == 0) {
+                asm volatile("" ::: "memory");   // (branches, as below; rows beyond the wave's are of no use)
 #pragma unroll
-                for (int j = 0; j < R; j++)
-                    if (j < w.nrows) ut[j] = s == 0 ? sd[j] : ut[j] + sd[j];
+                for (int j = 0; j < R; j++) ut[j] = sd[j];
+            } else if (halo_lane) {
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int j = 0; j < R; j++) ut[j] += sd[j];
             }
             if (s == steps) break;
             const T a = (T)coef[s], b = (T)coef[coef_stride + s];
@@ -967,28 +989,37 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_ppcg_resident(Tiles t, Fields<
 #pragma unroll
                     for (int i = 0; i < STRIP; i++) {
                         const int j = k * STRIP + i;
-                        const T q = co.apply(w, sd, sdb, j);
-                        if (w.out && j < w.nrows) rt[j] = rt[j] - q;
+                        rt[j] = rt[j] - co.apply(w, sd, sdb, j);   // (of no use outside the tile, but harmless)
                     }
                 }
             }
 #pragma unroll
             for (int k = 0; k < S; k++) {
                 if (k < w.mine) {
-                    T rv[STRIP], zv[STRIP];
+                    T rv[STRIP], nv[STRIP];
 #pragma unroll
                     for (int i = 0; i < STRIP; i++) rv[i] = rt[k * STRIP + i];
-                    if (PREC == PREC_BLOCK) fac.apply(w, co, k, rv, zv);
+                    if (PREC == PREC_BLOCK) {
+                        T zv[STRIP];
+                        fac.apply(w, co, k, rv, zv);
 #pragma unroll
-                    for (int i = 0; i < STRIP; i++) {
-                        const int j = k * STRIP + i;
-                        T n;
-                        if (PREC == PREC_BLOCK) n = a * sd[j] + b * zv[i];
-                        else if (PREC == PREC_DIAG) n = a * sd[j] + b * rv[i] * fac.mi(j);
-                        else n = a * sd[j] + b * rv[i];
-                        if (w.out && j < w.nrows) {
-                            sd[j] = n;
-                            ut[j] += n;
+                        for (int i = 0; i < STRIP; i++) nv[i] = a * sd[k * STRIP + i] + b * zv[i];
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < STRIP; i++) {
+                            const int j = k * STRIP + i;
+                            if (PREC == PREC_DIAG) nv[i] = a * sd[j] + b * rv[i] * fac.mi(j);
+                            else nv[i] = a * sd[j] + b * rv[i];
+                        }
+                    }
+                    w.cut(k, nv);
+                    if (w.out) {
+                        asm volatile("" ::: "memory");   // one branch per strip, not selects on every row
+#pragma unroll
+                        for (int i = 0; i < STRIP; i++) {
+                            const int j = k * STRIP + i;
+                            sd[j] = nv[i];
+                            ut[j] += nv[i];
                         }
                     }
                 }
@@ -1147,35 +1178,47 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_cheby_resident(Tiles t, Fields
                 for (int i = 0; i < STRIP; i++) {
                     const int j = k * STRIP + i;
                     const T a = co.apply(w, u, ub, j);
-                    v[j] = w.out && j < w.nrows ? u0[j] - a : T(0.0);
+                    v[j] = u0[j] - a;
                     if (check || last) {
                         w.store(bw, o, j, w.nrows, a);
                         w.store(br, o, j, w.nrows, v[j]);
                     }
                 }
+                w.cut(k, v, k * STRIP);
             }
         }
         if (check) {
 #pragma unroll
             for (int j = 0; j < R; j++) dd_add_prod(acc[0], (double)v[j], (double)v[j]);
+            acc[0] = w.owned(acc[0]);
         }
 #pragma unroll
         for (int k = 0; k < S; k++) {
             if (k < w.mine) {
-                T rv[STRIP], zv[STRIP];
+                T rv[STRIP], pv[STRIP];
 #pragma unroll
                 for (int i = 0; i < STRIP; i++) rv[i] = v[k * STRIP + i];
-                if (PREC == PREC_BLOCK) fac.apply(w, co, k, rv, zv);
+                if (PREC == PREC_BLOCK) {
+                    T zv[STRIP];
+                    fac.apply(w, co, k, rv, zv);
 #pragma unroll
-                for (int i = 0; i < STRIP; i++) {
-                    const int j = k * STRIP + i;
-                    T pv;
-                    if (PREC == PREC_BLOCK) pv = alpha * p[j] + beta * zv[i];
-                    else if (PREC == PREC_DIAG) pv = alpha * p[j] + beta * fac.mi(j) * rv[i];
-                    else pv = alpha * p[j] + beta * rv[i];
-                    if (w.out && j < w.nrows) {
-                        p[j] = pv;
-                        u[j] += pv;
+                    for (int i = 0; i < STRIP; i++) pv[i] = alpha * p[k * STRIP + i] + beta * zv[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < STRIP; i++) {
+                        const int j = k * STRIP + i;
+                        if (PREC == PREC_DIAG) pv[i] = alpha * p[j] + beta * fac.mi(j) * rv[i];
+                        else pv[i] = alpha * p[j] + beta * rv[i];
+                    }
+                }
+                w.cut(k, pv);
+                if (w.out) {
+                    asm volatile("" ::: "memory");   // one branch per strip, not selects on every row
+#pragma unroll
+                    for (int i = 0; i < STRIP; i++) {
+                        const int j = k * STRIP + i;
+                        p[j] = pv[i];
+                        u[j] += pv[i];
                     }
                 }
             }

@@ -41,7 +41,8 @@ constexpr int RES_HISTORY = 1024;   // iterations per launch at most
 // Words of the exchange buffers (all zero before the first launch).
 constexpr int RED_COPIES = 8;
 constexpr size_t RED_WORDS = 2 * (size_t)RED_COPIES * 8 * RES_MAX_WG;   // [slot][copy][word][workgroup]
-constexpr size_t COL_WORDS = 2 * (size_t)RES_MAX_WG * 2 * RES_WAVES * 64;    // [slot][workgroup][side][wave][64]
+constexpr int FACE_WORDS = 32;      // a column face of a wave: 16 rows in FP64, 32 in FP32
+constexpr size_t COL_WORDS = 2 * (size_t)RES_MAX_WG * 2 * RES_WAVES * FACE_WORDS;   // [slot][workgroup][side][wave][word]
 constexpr size_t ROW_WORDS = 2 * (size_t)RES_MAX_WG * 2 * 2 * 64; // [slot][workgroup][side][word][lane]
 constexpr size_t EXCHANGE_WORDS = RED_WORDS + COL_WORDS + ROW_WORDS + 16;
 
