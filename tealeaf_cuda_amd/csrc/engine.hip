@@ -192,8 +192,9 @@ struct Chunk {
     int max_blocks = 0;              // largest grid of any launch
     int last_grid = 0;               // grid of the latest launch
 
-    // resident runs: exchange words (in the field slab), the latest tag, and
+    // resident runs: exchange words, the latest tag, and
     // the values of a run's iterations (pinned, behind h_out)
+    double *res_mem = nullptr;       // null: the mesh has no runs
     res::Exchange res_x{};
     double *h_run = nullptr, *d_run = nullptr;
     double *h_coef = nullptr, *res_coef = nullptr;   // iteration coefficients: pinned staging, device copy
@@ -1096,6 +1097,7 @@ void release_all()
     if (g.d_partials) (void)hipFree(g.d_partials);
     if (g.h_out) (void)hipHostFree(g.h_out);
     if (g.d_scal) (void)hipFree(g.d_scal);
+    if (g.res_mem) (void)hipFree(g.res_mem);
     if (g.d_halo_buf) (void)hipFree(g.d_halo_buf);
     if (g.slab32) (void)hipFree(g.slab32);
     ws::net_free(g.ws_net);
@@ -1117,6 +1119,10 @@ void release_all()
                                  : launch(#KERNEL, KERNEL<PREC_NONE>, __VA_ARGS__))
 
 }  // namespace
+
+namespace {
+int cu_count();
+}
 
 EXPORT void initialise_cuda_(int *x_min, int *x_max, int *y_min, int *y_max)
 {
@@ -1159,17 +1165,21 @@ EXPORT void initialise_cuda_(int *x_min, int *x_max, int *y_min, int *y_max)
     HIP_OK(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
     const size_t field_elems = (size_t)g.pitch * (size_t)g.rows + 16;  // + slack, keeps 128-byte alignment
     const size_t field_stride = (field_elems + 31) / 32 * 32;
-    // behind the fields: the exchange words of resident runs (they start at zero too) and coefficients
-    const size_t slab_elems = field_stride * N_SLOTS + res::EXCHANGE_WORDS + (2 + RUN_VALUES) * res::RES_HISTORY;
-    HIP_OK(hipMalloc(&g.slab, slab_elems * sizeof(double)));
-    HIP_OK(hipMemsetAsync(g.slab, 0, slab_elems * sizeof(double), g.stream));
-    {
-        res::word_t *words = (res::word_t *)(g.slab + field_stride * N_SLOTS);
+    HIP_OK(hipMalloc(&g.slab, field_stride * N_SLOTS * sizeof(double)));
+    HIP_OK(hipMemsetAsync(g.slab, 0, field_stride * N_SLOTS * sizeof(double), g.stream));
+    // where the mesh may have resident runs: their exchange words (zero at first) and coefficients
+    res::Tiles tiles;
+    if (res::plan_tiles(tiles, g.nx, g.ny, g.h, g.pitch, 64, cu_count()) ||
+        res::plan_tiles(tiles, g.nx, g.ny, g.h, g.pitch, 32, cu_count())) {
+        const size_t n = res::EXCHANGE_WORDS + (2 + RUN_VALUES) * res::RES_HISTORY;
+        HIP_OK(hipMalloc(&g.res_mem, n * sizeof(double)));
+        HIP_OK(hipMemsetAsync(g.res_mem, 0, n * sizeof(double), g.stream));
+        res::word_t *words = (res::word_t *)g.res_mem;
         g.res_x.ctl = (unsigned *)words;
         g.res_x.red = words + 16;
         g.res_x.col = g.res_x.red + res::RED_WORDS;
         g.res_x.row = g.res_x.col + res::COL_WORDS;
-        g.res_coef = (double *)(words + res::EXCHANGE_WORDS);
+        g.res_coef = g.res_mem + res::EXCHANGE_WORDS;
         g.res_x.history = g.res_coef + 2 * res::RES_HISTORY;
     }
     for (int k = 1; k < N_SLOTS; k++) {
@@ -2744,8 +2754,8 @@ EXPORT void tea_leaf_ppcg_calc_p_kernel_cuda_(double *beta)
 //
 // Many iterations in one launch (resident.hpp) for every mesh whose fields fit
 // the chip (about 1500^2 cells in FP64, 2000^2 in FP32): a run wins from the
-// smallest to the largest of them (whole decks: 2.7 times at 10^2 cells, 4.9 at
-// 1000^2; at 1531 x 997, four strips per wave, PPCG 1.7 times).  TEA_RESIDENT=0
+// smallest to the largest of them (whole decks: 2.5 times at 10^2 cells, 4.8 at
+// 1000^2; at 1531 x 997, four strips per wave, PPCG 1.9 times).  TEA_RESIDENT=0
 // turns them off, and so does any switch that picks a form of the separate
 // kernels.
 namespace {
@@ -2757,7 +2767,7 @@ bool resident_tiles(res::Tiles &t)
                                   "TEA_CG_Z_FROM_R", "TEA_FUSED_INNER", "TEA_GRID_MAX", "TEA_SPECULATE",
                                   "TEA_SPEC_MARGIN", "TEA_PPCG_ITERATION", "TEA_INNER_PASSES"};
     const char *env = getenv("TEA_RESIDENT");
-    if (g.res_busy || (env && env[0] == '0')) return false;
+    if (!g.res_mem || g.res_busy || (env && env[0] == '0')) return false;
     for (const char *f : forms)
         if (getenv(f)) return false;
     return res::plan_tiles(t, g.nx, g.ny, g.h, g.fp32 ? g.pitch32 : g.pitch, g.fp32 ? 32 : 64, cu_count());

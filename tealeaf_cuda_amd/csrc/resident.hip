@@ -598,8 +598,8 @@ __device__ __forceinline__ bool replacement_due(const Stop &st, double q_ref, do
 // slower, 11.4 against 9.1 us per iteration of 1000^2 cells, with nothing to
 // run while a chain of FP64 operations waits).
 // Measured, FP64 without a preconditioner, a deck's whole run with its set-up,
-// against the separate kernels: 10^2 cells 1.31 (3.59) ms, 250^2 1.74 (8.82)
-// ms, 1000^2 4.67 (22.95) ms; per iteration 6 us at 250^2 (two exchanges'
+// against the separate kernels: 10^2 cells 1.38 (3.43) ms, 250^2 1.95 (10.15)
+// ms, 1000^2 5.18 (25.00) ms; per iteration 6 us at 250^2 (two exchanges'
 // latency), 9 at 1000^2 (that and FP64 issue).
 template <typename T, int PREC, int S>
 __global__ __launch_bounds__(RES_BLOCK, 2) void k_cg_resident(Tiles t, Fields<T> f, Exchange x, int with_p,
@@ -765,10 +765,10 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_cg_resident(Tiles t, Fields<T>
 // more than the reads).  An inner step is one neighbour exchange (no
 // all-reduce): bound by its latency on small meshes, by issue on the largest.
 // Measured, FP64, a deck's whole run with its CG steps and set-up, against the
-// separate passes: 512^2 block Jacobi, 10 inner steps 4.14 (9.48) ms; 1531 x
-// 997 jac_diag, halo depth 2, to the FP64 true residual 9.14 (17.21) ms.  At
-// four strips per wave an inner step takes 6.6 us: 4.7 of issue (with selects
-// per row instead of branches per strip, 5.2), 0.8 before the exchange is in.
+// separate passes: 512^2 block Jacobi, 10 inner steps 4.56 (11.11) ms; 1531 x
+// 997 jac_diag, halo depth 2, to the FP64 true residual 10.89 (20.65) ms (with
+// selects per row instead of branches per strip 9% more).  There, four strips
+// per wave, two thirds of an inner step are issue and a fifth the exchange.
 template <typename T, int PREC, int S>
 __global__ __launch_bounds__(RES_BLOCK, 2) void k_ppcg_resident(Tiles t, Fields<T> f, Exchange x, int from_inner,
                                                                 int with_p, double beta_in, double rro,
@@ -1132,7 +1132,7 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_ppcg_resident(Tiles t, Fields<
 // the iterations whose norm the caller tests.  w and r are written out where
 // the run may end (the reference leaves the last iteration's in their fields).
 // Measured, FP64, 1533 x 1021 cells, a deck's whole run with its CG steps and
-// set-up, against the separate passes: 4.37 (15.01) ms.
+// set-up, against the separate passes: 4.11 (14.19) ms.
 template <typename T, int PREC, int S>
 __global__ __launch_bounds__(RES_BLOCK, 2) void k_cheby_resident(Tiles t, Fields<T> f, Exchange x,
                                                                  const double *__restrict__ coef, int coef_stride,
