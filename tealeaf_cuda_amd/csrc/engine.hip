@@ -2945,9 +2945,12 @@ EXPORT int tea_engine_cg_run(int with_p, double beta, double rro, int max_its, c
     res::Tiles t;
     if (max_its < 1 || !resident_tiles(t)) return 0;
     g.calls++;
-    g.pending_w = 0;   // rewritten
+    const int w_owed = g.pending_w;   // rewritten, if the run starts
+    g.pending_w = 0;
     settle_pending();
-    return BY_PRECISION(cg_run_impl, t, with_p, beta, rro, max_its, stop, pw, rrn);
+    const int n = BY_PRECISION(cg_run_impl, t, with_p, beta, rro, max_its, stop, pw, rrn);
+    if (n == 0) g.pending_w = w_owed;
+    return n;
 }
 
 EXPORT int tea_engine_ppcg_run(int from_inner, int with_p, double beta, double rro, double theta, int inner_steps,
@@ -2961,9 +2964,12 @@ EXPORT int tea_engine_ppcg_run(int from_inner, int with_p, double beta, double r
     res::Tiles t;
     if (max_its < 1 || inner_steps > res::RES_HISTORY || !resident_tiles(t)) return 0;
     g.calls++;
+    const int w_owed = from_inner ? 0 : g.pending_w;   // dropped, if the run starts
     if (!from_inner) drop_w_settle_rest();
-    return BY_PRECISION(ppcg_run_impl, t, from_inner, with_p, beta, rro, theta, inner_steps, max_its, stop, values,
-                        at_ur, rrn_end);
+    const int n = BY_PRECISION(ppcg_run_impl, t, from_inner, with_p, beta, rro, theta, inner_steps, max_its, stop,
+                               values, at_ur, rrn_end);
+    if (n == 0 && w_owed) g.pending_w = w_owed;
+    return n;
 }
 
 EXPORT int tea_engine_cheby_run(int step, int n, int check_from, double error, double target, int max_its, double *rr)
@@ -2978,9 +2984,12 @@ EXPORT int tea_engine_cheby_run(int step, int n, int check_from, double error, d
     res::Tiles t;
     if (!resident_tiles(t)) return 0;
     g.calls++;
-    g.pending_cheby = 0;   // the iterations form w and r again
+    const auto owed = g.pending_cheby;   // the iterations form w and r again, if the run starts
+    g.pending_cheby = 0;
     settle_pending();
-    return BY_PRECISION(cheby_run_impl, t, k, n, check_from, error, target, max_its, rr);
+    const int done = BY_PRECISION(cheby_run_impl, t, k, n, check_from, error, target, max_its, rr);
+    if (done == 0) g.pending_cheby = owed;
+    return done;
 }
 
 // =============================================================================
