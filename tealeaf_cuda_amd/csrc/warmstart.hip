@@ -667,28 +667,81 @@ __global__ void k_out_bwd(const float *__restrict__ g6, const float *__restrict_
 constexpr int WG_PARTS = 512;
 
 // Layer 6 weight and bias gradients, dW6[tap][ci] = sum_p a5[p + tap][ci] g6[p]
-// and db6 = sum_p g6[p], summed over the input pixels q = p + tap (a5 and g6
-// are zero on the border).  One product per 72 loaded values, so the pass is
-// bound by reading a5 once: a lane holds 8 channels of one pixel column
-// (one 16-byte load per pixel), marches down a run of rows and keeps the 3x3
-// window of g6 and the 72 sums in registers; 4 lanes cover a pixel, a wave 16
-// columns.  32 x 128 x 128 pixels: 1060 us with one thread per weight walking
-// every pixel, 20 us here.  tasks: (image, 16 columns, run of rows).
-__global__ __launch_bounds__(BLOCK) void k_out_wgrad(const __bf16 *__restrict__ a5, const float *__restrict__ g6,
-                                                     float *__restrict__ part, int H, int W, int rows, int nruns,
-                                                     long tasks)
+// and db6 = sum_p g6[p].
+//
+// The weights are summed over the input pixels q = p + tap (a5 and g6 are zero
+// on the border).  One product per 72 loaded values, so that part is bound by
+// reading a5 once: a lane holds 8 channels of one pixel column (one 16-byte load
+// per pixel), marches down a run of rows and keeps the 3x3 window of g6 and the
+// 72 sums in registers; 4 lanes cover a pixel, a wave 16 columns.  32 x 128 x 128
+// pixels: 1060 us with one thread per weight walking every pixel, 20 us here (29
+// with the bias).  tasks: (image, 16 columns, run of rows).
+//
+// Under the energy loss g6 is made of fluxes that cancel in db6 (the sum of
+// |g6| is 13 to 7000 times |db6| over 40 batches of 32 x 128 x 128), so the order
+// of its FP32 sum shows in db6, and the order is fixed: BIAS_RUNS runs of
+// consecutive pixels, each summed first pixel to last, then the runs' sums first
+// to last (k_sum_runs).
+// One wave per run, in the workgroups after the first `wparts`, beside the others'
+// reads of a5: it loads 64 pixels side by side and adds them one by one out of its
+// lanes.  Bound by that chain (35 us with one such load under way instead of eight).
+constexpr int BIAS_RUNS = 256;
+
+// s + v of lane 0 + v of lane 1 + ... of the first n lanes, in that order
+__device__ __forceinline__ float add_in_order(float s, float v, int n)
 {
-    constexpr int NOUT = TAPS * CH + 1, NW = BLOCK / 64;
+    if (n == 64) {
+#pragma unroll
+        for (int k = 0; k < 64; k++) s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+    } else {
+        for (int k = 0; k < n; k++) s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+    }
+    return s;
+}
+
+__global__ __launch_bounds__(BLOCK) void k_out_wgrad(const __bf16 *__restrict__ a5, const float *__restrict__ g6,
+                                                     float *__restrict__ part, float *__restrict__ runs, int B, int H,
+                                                     int W, int rows, int nruns, long tasks, int wparts)
+{
+    constexpr int NOUT = TAPS * CH, NW = BLOCK / 64, AHEAD = 8;
     __shared__ float lds[NW][NOUT];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if ((int)blockIdx.x >= wparts) {
+        const int c = ((int)blockIdx.x - wparts) * NW + wave;
+        if (c >= BIAS_RUNS) return;
+        // (pixels are counted in 32 bits: 2^31 of them would be 137 GB per layer)
+        const long n = (long)B * H * W;
+        const unsigned p1 = (unsigned)(n * (c + 1) / BIAS_RUNS);
+        auto pixel = [&](unsigned p) {
+            if (p >= p1) return 0.0f;
+            const unsigned row = p / (unsigned)W, b = row / (unsigned)H;
+            return g6[padded((int)b, (int)(row - b * H), (int)(p - row * W), H, W)];
+        };
+        unsigned p = (unsigned)(n * c / BIAS_RUNS);
+        float s = 0.0f, next[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) next[u] = pixel(p + u * 64 + lane);
+        for (; p < p1; p += AHEAD * 64) {
+            float v[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) {
+                v[u] = next[u];
+                next[u] = pixel(p + (AHEAD + u) * 64 + lane);   // under way while these are added
+            }
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) s = add_in_order(s, v[u], (int)min(64l, max(0l, (long)p1 - p - u * 64)));
+        }
+        if (lane == 0) runs[c] = s;
+        return;
+    }
     const int q = lane & 3, px = lane >> 2;
     const int cols = W / 16;
-    float acc[TAPS][8], accb = 0.0f;
+    float acc[TAPS][8];
 #pragma unroll
     for (int t = 0; t < TAPS; t++)
 #pragma unroll
         for (int i = 0; i < 8; i++) acc[t][i] = 0.0f;
-    for (long task = (long)blockIdx.x * NW + wave; task < tasks; task += (long)gridDim.x * NW) {
+    for (long task = (long)blockIdx.x * NW + wave; task < tasks; task += (long)wparts * NW) {
         const int run = (int)(task % nruns);
         const int xg = (int)((task / nruns) % cols), b = (int)(task / nruns / cols);
         const int x = xg * 16 + px, y0 = run * rows, y1 = min(y0 + rows, H);
@@ -707,7 +760,6 @@ __global__ __launch_bounds__(BLOCK) void k_out_wgrad(const __bf16 *__restrict__ 
                 gw[2][j] = g6[padded(b, y + 1, x - 1 + j, H, W)];
             }
             const bf16x8 a = *(const bf16x8 *)(a5 + padded(b, y, x, H, W) * CH + q * 8);
-            accb += gw[1][1];
 #pragma unroll
             for (int t = 0; t < TAPS; t++) {
                 const float g = gw[2 - t / 3][2 - t % 3];   // g6 at p = q - tap
@@ -722,18 +774,27 @@ __global__ __launch_bounds__(BLOCK) void k_out_wgrad(const __bf16 *__restrict__ 
         for (int t = 0; t < TAPS; t++)
 #pragma unroll
             for (int i = 0; i < 8; i++) acc[t][i] += __shfl_xor(acc[t][i], off, 64);
-        accb += __shfl_xor(accb, off, 64);
     }
     if (px == 0) {
 #pragma unroll
         for (int t = 0; t < TAPS; t++)
 #pragma unroll
             for (int i = 0; i < 8; i++) lds[wave][t * CH + q * 8 + i] = acc[t][i];
-        if (q == 0) lds[wave][TAPS * CH] = accb;
     }
     __syncthreads();
     for (int e = threadIdx.x; e < NOUT; e += BLOCK)
         part[(long)blockIdx.x * NOUT + e] = (lds[0][e] + lds[1][e]) + (lds[2][e] + lds[3][e]);
+}
+
+// db6 from the runs' sums, in order.
+__global__ __launch_bounds__(64) void k_sum_runs(const float *__restrict__ runs, float *__restrict__ dst)
+{
+    float s = 0.0f, v[BIAS_RUNS / 64];
+#pragma unroll
+    for (int k = 0; k < BIAS_RUNS / 64; k++) v[k] = runs[k * 64 + threadIdx.x];
+#pragma unroll
+    for (int k = 0; k < BIAS_RUNS / 64; k++) s = add_in_order(s, v[k], 64);
+    if (threadIdx.x == 0) *dst = s;
 }
 
 // Weight and bias gradients of a 32-channel layer: dW[tap][ci][co] =
@@ -1173,9 +1234,11 @@ int backward_pass(Trainer *t, const float *samples)
         const int nruns = (H + rows - 1) / rows;
         const long tasks = cols * nruns;
         const int parts = (int)std::min<long>(WG_PARTS, (tasks + 3) / 4);
-        hipLaunchKernelGGL(k_out_wgrad, dim3(parts), dim3(BLOCK), 0, s, t->acts.a[5], t->g6, t->part, H, W, rows,
-                           nruns, tasks);
-        sum_parts(t->part, parts, TAPS * CH + 1, t->grad + OFF_W6, s);
+        float *runs = t->part + (long)WG_PARTS * TAPS * CH;
+        hipLaunchKernelGGL(k_out_wgrad, dim3(parts + BIAS_RUNS / (BLOCK / 64)), dim3(BLOCK), 0, s, t->acts.a[5],
+                           t->g6, t->part, runs, B, H, W, rows, nruns, tasks, parts);
+        hipLaunchKernelGGL(k_sum_runs, dim3(1), dim3(64), 0, s, runs, t->grad + OFF_B6);
+        sum_parts(t->part, parts, TAPS * CH, t->grad + OFF_W6, s);
     }
     hipLaunchKernelGGL(k_out_bwd, dim3(nblocks(npix)), dim3(BLOCK), 0, s, t->g6, t->net.w6, t->acts.a[5], t->g[0],
                        B, H, W);
