@@ -1106,13 +1106,15 @@ int march_run_rows(int H, int W, int B, int rows)
 
 // The marching layers (k_first_conv32_march, k_conv32_march,
 // k_conv_out_march) for one image where the height is a multiple of 16,
-// unless TEA_WS_MARCH=0.
-template <int ROWS> void forward_rows(const Net &net, const Acts &a, const float *planes, int npl, hipStream_t stream)
+// unless TEA_WS_MARCH=0.  Not before a backward pass (layers_too): the march keeps
+// layer 1's output in LDS, and the gradients of layers 1 and 2 read it from memory.
+template <int ROWS>
+void forward_rows(const Net &net, const Acts &a, const float *planes, int npl, hipStream_t stream, bool layers_too)
 {
     const dim3 grid(a.W / 64, a.H / ROWS, a.B), block(ROWS * 64);
     const bf16x8 *pk = (const bf16x8 *)net.packed;
     const char *env = getenv("TEA_WS_MARCH");
-    const bool march = ROWS == 16 && a.B == 1 && !(env && env[0] == '0');
+    const bool march = ROWS == 16 && a.B == 1 && !layers_too && !(env && env[0] == '0');
     int run_rows = march_run_rows(a.H, a.W, a.B, ROWS);
     // TEA_WS_MARCH_ROWS=<rows> sets the run length (tests march several blocks on small images)
     if (const char *s = getenv("TEA_WS_MARCH_ROWS")) {
@@ -1144,11 +1146,11 @@ template <int ROWS> void forward_rows(const Net &net, const Acts &a, const float
 
 // Inference takes workgroups of 16 rows where the height allows it: a smaller
 // share of re-read halo rows (18/16 against 10/8 per staged window).
-void forward(const Net &net, const Acts &a, const float *planes, int npl, hipStream_t stream)
+void forward(const Net &net, const Acts &a, const float *planes, int npl, hipStream_t stream, bool layers_too)
 {
-    if (a.H % 16 == 0) forward_rows<16>(net, a, planes, npl, stream);
-    else if (conv_rows(a.H) == 8) forward_rows<8>(net, a, planes, npl, stream);
-    else forward_rows<4>(net, a, planes, npl, stream);
+    if (a.H % 16 == 0) forward_rows<16>(net, a, planes, npl, stream, layers_too);
+    else if (conv_rows(a.H) == 8) forward_rows<8>(net, a, planes, npl, stream, layers_too);
+    else forward_rows<4>(net, a, planes, npl, stream, layers_too);
 }
 
 }  // namespace ws
@@ -1202,10 +1204,10 @@ void destroy(Trainer *t)
     delete t;
 }
 
-int forward_pass(Trainer *t, const float *samples)
+int forward_pass(Trainer *t, const float *samples, bool layers_too)
 {
     ws::im2col(t->acts, samples, ws::NPLANES, t->stream);
-    ws::forward(t->net, t->acts, samples, ws::NPLANES, t->stream);
+    ws::forward(t->net, t->acts, samples, ws::NPLANES, t->stream, layers_too);
     WS_OK(hipGetLastError());
     return 0;
 }
@@ -1365,7 +1367,7 @@ EXPORT int tea_ws_trainer_forward(void *h, const float *samples, float *out_host
 {
     Trainer *t = (Trainer *)h;
     if (!t || !samples || !out_host) return ws_fail("tea_ws_trainer_forward: null argument");
-    if (forward_pass(t, samples)) return -1;
+    if (forward_pass(t, samples, false)) return -1;
     WS_OK(hipMemcpyAsync(out_host, t->acts.out, (size_t)t->B * t->H * t->W * sizeof(float), hipMemcpyDeviceToHost,
                          t->stream));
     WS_OK(hipStreamSynchronize(t->stream));
@@ -1376,7 +1378,7 @@ EXPORT int tea_ws_trainer_gradient(void *h, const float *samples, float *grad_ho
 {
     Trainer *t = (Trainer *)h;
     if (!t || !samples || !grad_host) return ws_fail("tea_ws_trainer_gradient: null argument");
-    if (forward_pass(t, samples) || backward_pass(t, samples)) return -1;
+    if (forward_pass(t, samples, true) || backward_pass(t, samples)) return -1;
     WS_OK(hipMemcpyAsync(grad_host, t->grad, ws::NPARAM * sizeof(float), hipMemcpyDeviceToHost, t->stream));
     WS_OK(hipStreamSynchronize(t->stream));
     return read_loss(t, loss);
@@ -1386,7 +1388,7 @@ EXPORT int tea_ws_trainer_step(void *h, const float *samples, float lr, double *
 {
     Trainer *t = (Trainer *)h;
     if (!t || !samples) return ws_fail("tea_ws_trainer_step: null argument");
-    if (forward_pass(t, samples) || backward_pass(t, samples)) return -1;
+    if (forward_pass(t, samples, true) || backward_pass(t, samples)) return -1;
     if (loss && read_loss(t, loss)) return -1;
     t->step++;
     const float b1 = 0.9f, b2 = 0.999f;

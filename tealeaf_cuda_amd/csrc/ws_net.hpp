@@ -90,8 +90,10 @@ void acts_free(Acts &a);
 // Training: the im2col image x1 of the feature planes (planes[b][f][y][x],
 // npl FP32 planes per image, features f = 0..2), for layer 1's weight gradient.
 void im2col(const Acts &a, const float *planes, int npl, hipStream_t stream);
-// Layers 1..6 from the feature planes; writes a.a[1..5] and a.out.
-void forward(const Net &net, const Acts &a, const float *planes, int npl, hipStream_t stream);
+// Layers 1..6 from the feature planes; writes a.out, and with layers_too every
+// layer's output a.a[1..5] (for a backward pass).
+void forward(const Net &net, const Acts &a, const float *planes, int npl, hipStream_t stream,
+             bool layers_too = false);
 
 }  // namespace ws
 

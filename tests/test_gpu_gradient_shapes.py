@@ -60,8 +60,8 @@ def test_gradient_at_odd_shapes(shape):
         t.close()
 
 
-SHAPES = [(1, 4, 64, 0), (1, 68, 128, 32), (2, 80, 192, 32), (4, 32, 64, 0), (8, 128, 128, 0),
-          (64, 8, 64, 0)]
+SHAPES = [(1, 4, 64, 0), (1, 68, 128, 32), (2, 80, 192, 32), (4, 32, 64, 0), (1, 64, 64, 0), (1, 128, 128, 0),
+          (8, 128, 128, 0), (64, 8, 64, 0)]
 
 
 @pytest.mark.parametrize("loss", ["mse", "energy"])
