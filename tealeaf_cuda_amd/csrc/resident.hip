@@ -874,14 +874,13 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_ppcg_resident(Tiles t, Fields<
             w.template part<2>(sh, acc);
             __syncthreads();
             w.template post_total<2>(sh);
-            // while the sums travel: p and rstore = r
+            // while the sums travel: rstore = r
 #pragma unroll
             for (int j = 0; j < R; j++) {
                 if (KEEP) {
                     pk[KEEP ? j : 0] = sd[j];
                     rsk[KEEP ? j : 0] = ut[j];
                 } else {
-                    w.store(bp, o, j, w.nrows, sd[j]);
                     w.store(brs, o, j, w.nrows, ut[j]);
                 }
             }
@@ -892,6 +891,12 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_ppcg_resident(Tiles t, Fields<
             w.template collect_total<2>(sh);
             __syncthreads();
             if (sh.bad) break;
+            // p goes to memory only now: the neighbours read its outer cells there
+            // when their run starts, and their sums, which have come, follow those reads
+            if (!KEEP) {
+#pragma unroll
+                for (int j = 0; j < R; j++) w.store(bp, o, j, w.nrows, sd[j]);
+            }
             pw = w.total(sh, 0);
             rz = w.total(sh, 1);
             alpha = (T)(rz / pw);
