@@ -1341,7 +1341,10 @@ Run::Solve Run::iterate(double initial_residual_sq, double eps)
             cg_p_pending = run_next == run_rrn.size();   // else applied inside the run
             cg_beta_pending = beta;
             if (rel.on) {
-                if (replacement_due(rrn)) flush_cg_p();   // calc_p comes first
+                if (replacement_due(rrn)) {
+                    if (run_next < run_rrn.size()) fail("a run of CG iterations went past a residual replacement");
+                    flush_cg_p();   // calc_p comes first
+                }
                 // a replaced r reaches z at the next cg_calc_ur
                 if (reliable_step(rrn, false, nullptr)) converged = true;
             }
