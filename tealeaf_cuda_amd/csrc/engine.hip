@@ -200,6 +200,7 @@ struct Chunk {
     double *h_coef = nullptr, *res_coef = nullptr;   // iteration coefficients: pinned staging, device copy
     int res_coef_at = -1, res_coef_n = 0;            // the ones the device copy holds
     bool res_busy = false;   // a run found part of the chip taken: no more of them (finding out costs 0.2 s)
+    int res_started = 0;     // runs launched while TEA_RESIDENT_TAKEN is set
 
     double *d_halo_buf = nullptr;    // staging for pack / unpack
     size_t halo_buf_elems = 0;
@@ -2838,10 +2839,17 @@ const double *resident_coefs(int k0, int n)
 }
 
 // Launches a run, waits for it and returns its iterations; 0 if it did not
-// start or on an error.
+// start or on an error.  TEA_RESIDENT_TAKEN=<n> (tests): the runs after the
+// chunk's first n find their workgroups' verdict given, as if some of them had
+// waited in vain for the others.
 template <typename L> int resident_run(const char *name, L launch_run)
 {
     hipError_t err;
+    const char *taken = getenv("TEA_RESIDENT_TAKEN");
+    if (taken && g.res_started++ >= atoi(taken)) {
+        err = hipMemsetD32Async((hipDeviceptr_t)(g.res_x.ctl + 1), (int)res::VERDICT_ABORT, 1, g.stream);
+        if (err != hipSuccess) { die("hipMemsetD32Async failed: %s", hipGetErrorString(err)); return 0; }
+    }
     {
         Timed timed(name);
         err = launch_run(g.d_run + 4, (res::Outcome *)g.d_run);
@@ -2851,7 +2859,12 @@ template <typename L> int resident_run(const char *name, L launch_run)
     if (err != hipSuccess) { die("hipStreamSynchronize failed: %s", hipGetErrorString(err)); return 0; }
     if (g_profile_table && g.prof.on) g.prof.drain(false);
     const int n = ((const res::Outcome *)g.h_run)->iterations;
-    if (n == -1) { g.res_busy = true; return 0; }
+    if (n == -1) {
+        g.res_busy = true;
+        fprintf(stderr, "tea_engine: part of the GPU is taken by other work: solver iterations go back to separate "
+                        "launches (slower) until the engine is initialised again\n");
+        return 0;
+    }
     if (n < 0) { die("%s: an exchange among the workgroups timed out", name); return 0; }
     return n;
 }

@@ -20,7 +20,6 @@ constexpr long long EXCHANGE_TICKS = 1000000000;  // 10 s
 // for (an iteration of 1000^2 cells: 12.2 us without the waits and with one
 // copy of the sums, 10.0 with both, PREC_NONE, 6 strips in 4 waves).
 constexpr int FIRST_LOOK = 24, NEXT_LOOK = 2;
-enum { VERDICT_NONE = 0, VERDICT_GO = 1, VERDICT_ABORT = 2 };
 
 __device__ __forceinline__ word_t load_word(const word_t *p)
 {

@@ -47,6 +47,7 @@ constexpr size_t ROW_WORDS = 2 * (size_t)RES_MAX_WG * 2 * 2 * 64; // [slot][work
 constexpr size_t EXCHANGE_WORDS = RED_WORDS + COL_WORDS + ROW_WORDS + 16;
 
 typedef unsigned long long word_t;
+enum : unsigned { VERDICT_NONE = 0, VERDICT_GO = 1, VERDICT_ABORT = 2 };   // whether all workgroups are resident
 
 struct Exchange {
     word_t *red, *col, *row;

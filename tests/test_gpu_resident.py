@@ -139,3 +139,82 @@ def test_decks_without_runs(name, oracle_so, driver_built, oracle_env, monkeypat
     assert gpu.exact_error == cpu.exact_error
     for a, b in zip(gpu.summaries, cpu.summaries):
         assert a.values() == b.values(), (a, b)
+
+
+# A run that does not start (part of the chip is taken: the workgroups' verdict is given from the host), after
+# calls that leave fields owed, then the single calls: what they leave is what they leave without it.
+NOT_STARTED = {
+    "cg": [(lambda e: e.cg_begin_ur(True, 0.3, 0.9), lambda e: e.cg_run(True, 0.61, 0.8, 5, NEVER),
+            lambda e: (e.cg_begin_ur(True, 0.61, 0.8), e.calc_2norm(2))),
+           (lambda e: e.cg_begin_ur(True, 0.3, 0.9), lambda e: e.cg_run(True, 0.61, 0.8, 5, NEVER), lambda e: None)],
+    "ppcg": [(lambda e: e.ppcg_iteration(True, 0.3, 1.7, 4),
+              lambda e: e.ppcg_run(False, True, 0.45, 0.8, 1.7, 5, 3, NEVER),
+              lambda e: (e.ppcg_iteration(True, 0.45, 1.7, 5), e.calc_2norm(1))),
+             (lambda e: e.ppcg_iteration(True, 0.3, 1.7, 4),
+              lambda e: e.ppcg_run(False, True, 0.45, 0.8, 1.7, 5, 3, NEVER), lambda e: None),
+             (lambda e: e.ppcg_begin_ur(True, 0.3, 1.7), lambda e: e.ppcg_run(True, False, 0.0, 0.8, 1.7, 4, 2, NEVER),
+              lambda e: (e.ppcg_inner_n(1, 4), e.ppcg_end(), e.calc_2norm(1))),
+             (lambda e: e.ppcg_begin_ur(True, 0.3, 1.7), lambda e: e.ppcg_run(True, False, 0.0, 0.8, 1.7, 4, 2, NEVER),
+              lambda e: None)],
+    "chebyshev": [(lambda e: (e.cheby_init(ALPHAS, BETAS, 1.3), e.cheby_iterate_n(1, 3)),
+                   lambda e: e.cheby_run(4, 4, 10**6, 1.0, 0.0, 5), lambda e: (e.cheby_iterate_n(4, 2), e.calc_2norm(1))),
+                  (lambda e: (e.cheby_init(ALPHAS, BETAS, 1.3), e.cheby_iterate_n(1, 3)),
+                   lambda e: e.cheby_run(4, 4, 10**6, 1.0, 0.0, 5), lambda e: None)],
+}
+
+
+@pytest.mark.parametrize("bits", [64, 32])
+@pytest.mark.parametrize("prec", ["none", "jac_diag", "jac_block"])
+@pytest.mark.parametrize("solver", sorted(NOT_STARTED))
+def test_run_that_does_not_start(solver, prec, bits, oracle_so, oracle_env, monkeypatch, tmp_path, capfd):
+    oracle_env("dot2")
+    monkeypatch.setenv("TEA_RESIDENT_TAKEN", "0")
+    g, c = Engine(), Engine(oracle_so)
+    try:
+        for k, (before, run, after) in enumerate(NOT_STARTED[solver]):
+            print(f"[gpu resident] not started: {solver}/{prec} fp{bits}, {k}", flush=True)
+            for e in (g, c):
+                _prepare(e, tmp_path, solver, prec, nx=125, ny=71, halo=2)
+                if bits == 32:
+                    e.set_precision(32)
+                    e.mp_setup()
+            rand = _randomise if bits == 64 else _randomise32
+            rand((g, c), seed=k)
+            for e in (g, c):
+                e.cg_init()
+                if solver == "ppcg":
+                    e.ppcg_init_constants(ALPHAS, BETAS)
+            rand((g, c), seed=100 + k)
+            outs = []
+            for e in (g, c):
+                out = [before(e)]
+                if e is g:
+                    got = run(e)
+                    assert not (got[0] if isinstance(got, tuple) else got)
+                    assert "part of the GPU is taken" in capfd.readouterr().err
+                out.append(after(e))
+                outs.append(repr(out))
+            assert outs[0] == outs[1], k
+            for fid in range(1, 20):
+                if bits == 32 and fid in (rt.XFIELD_CP, rt.XFIELD_BFP):
+                    continue
+                a, b = (e.get_field(fid) if bits == 64 else e.get_field32(fid) for e in (g, c))
+                assert np.array_equal(a, b, equal_nan=True), f"case {k}: field {fid}"
+    finally:
+        g.finalize()
+        c.finalize()
+
+
+@pytest.mark.parametrize("runs", [0, 1, 2])
+@pytest.mark.parametrize("name", ["cg_block", "cheby_diag", "ppcg_diag_h2", "mixed_cg_block", "mixed_ppcg_diag_h2",
+                                  "refined_fp64_ppcg_block", "mixed_cheby_block"])
+def test_decks_whose_runs_stop_starting(name, runs, oracle_so, driver_built, oracle_env, monkeypatch, tmp_path):
+    oracle_env("dot2")
+    monkeypatch.setenv("TEA_RESIDENT_TAKEN", str(runs))
+    print(f"[gpu resident] deck {name}, {runs} runs start", flush=True)
+    path = _deck(**DECKS[name]).write(tmp_path / "tea.in")
+    gpu, cpu = run_deck(path), run_deck(path, backend=oracle_so)
+    assert gpu.iterations == cpu.iterations and gpu.refinements == cpu.refinements
+    assert gpu.ppcg_inner == cpu.ppcg_inner and gpu.exact_error == cpu.exact_error
+    for a, b in zip(gpu.summaries, cpu.summaries):
+        assert a.values() == b.values(), (a, b)
