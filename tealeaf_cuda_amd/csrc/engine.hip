@@ -514,7 +514,8 @@ bool collect(double *dst, int slot, int n)
             ask = clock::now() + patience;
         }
     }
-    if (g_profile_table && g.prof.on) g.prof.drain(false);   // so the table at exit needs no HIP call
+    // so the table at exit needs no HIP call (the values come before their launch is retired)
+    if (g_profile_table && g.prof.on) g.prof.drain(true);
     return true;
 }
 bool fetch(double *dst, int n) { return finish(0, n, nullptr) && collect(dst, 0, n); }

@@ -19,6 +19,8 @@ oracle where the oracle finishes in seconds.
 from __future__ import annotations
 
 import json
+import subprocess
+import sys
 
 import pytest
 
@@ -176,3 +178,26 @@ def test_profiler_on_table(tmp_path):
     assert all(v >= 0.0 for v in table.values()) and sum(table.values()) > 0.0
     assert list(table) == sorted(table)
     assert "Profiler Output" in (tmp_path / "tea.out").read_text()   # the driver's own table
+
+
+def test_profile_table_at_exit_has_the_last_launch(tmp_path):
+    """A program that ends without releasing its chunk: the table holds every
+    launch up to the last returned value, the reduction behind it included."""
+    print("[gpu configs] profiler_on table of a chunk that is not released", flush=True)
+    deck = Deck(x_cells=64, y_cells=64, solver="cg", preconditioner="none", profiler_on=True,
+                states=standard_states())
+    path = deck.write(tmp_path / "tea.in")
+    program = f"""
+import ctypes, sys
+sys.path.insert(0, {str(REPO)!r})
+from tealeaf_cuda_amd import Engine
+e = Engine()
+e.initialise({str(path)!r}, 64, 64)
+e.field_summary()
+ctypes.CDLL(None).exit(0)
+"""
+    run = subprocess.run([sys.executable, "-c", program], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True,
+                         timeout=100)
+    assert run.returncode == 0, run.stderr[-2000:]
+    rows = [line.rpartition(" : ")[0].strip() for line in run.stdout.splitlines()]
+    assert "field_summary" in rows and "finish" in rows, run.stdout
