@@ -89,6 +89,15 @@ def test_production_shape_bitwise(precision, oracle_so, driver_built, oracle_env
     assert all(e < (1e-10 if precision == "fp32" else 1e-8) for e in gpu.exact_error)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_production_shape_bitwise_in_passes(precision, oracle_so, driver_built, oracle_env, monkeypatch, tmp_path):
+    """The same without runs in one launch, which 1024^2 otherwise takes: the
+    streaming passes, the deferred end and the inner passes queued ahead, as
+    at 4096^2."""
+    monkeypatch.setenv("TEA_RESIDENT", "0")
+    test_production_shape_bitwise(precision, oracle_so, driver_built, oracle_env, tmp_path)
+
+
 LAYOUT = [StateSpec(100.0, 0.0001), StateSpec(0.1, 25.0, "rectangle", 0.0, 1.0, 1.0, 2.0),
           StateSpec(0.1, 0.1, "rectangle", 1.0, 6.0, 1.0, 2.0), StateSpec(0.1, 0.1, "rectangle", 5.0, 6.0, 1.0, 8.0),
           StateSpec(5.0, 2.0, "circle", 3.0, 0.0, 6.0, 0.0, 1.5)]

@@ -113,6 +113,39 @@ def test_runs_bitwise_tall_tiles(solver, prec, bits, ny, oracle_so, oracle_env, 
         c.finalize()
 
 
+# several rows of tiles with several strips per wave (p, u, r and rstore of PPCG then stay in memory), the last row
+# of tiles and the last strip short; the second run of a solve; fewer inner steps than strips per wave
+MORE_PPCG = [("never", lambda e, s: (e.ppcg_run(False, False, 0.0, 0.8, 1.7, 3, 2, s),
+                                     e.ppcg_run(False, True, 0.45, 0.8, 1.7, 3, 2, s))),
+             ("never", lambda e, s: e.ppcg_run(False, True, 0.45, 0.8, 1.7, 1, 3, s))]
+
+
+@pytest.mark.parametrize("bits,nx,ny", [(64, 1235, 390), (32, 1235, 775)])      # 2 and 3 strips
+@pytest.mark.parametrize("solver,prec", [("ppcg", "none"), ("ppcg", "jac_diag"), ("ppcg", "jac_block"),
+                                         ("cg", "jac_diag"), ("cg", "jac_block"), ("chebyshev", "none")])
+def test_runs_bitwise_on_a_grid_of_tiles(solver, prec, bits, nx, ny, oracle_so, oracle_env, tmp_path):
+    oracle_env("dot2")
+    g, c = Engine(), Engine(oracle_so)
+    try:
+        runs = RUNS[solver] + (MORE_PPCG if solver == "ppcg" else [])
+        _check(g, c, solver, prec, bits, nx, ny, runs, tmp_path)
+    finally:
+        g.finalize()
+        c.finalize()
+
+
+@pytest.mark.parametrize("bits,ny", [(64, 127), (32, 250)])                     # 4 and 8 strips
+@pytest.mark.parametrize("prec", ["none", "jac_diag", "jac_block"])
+def test_ppcg_runs_bitwise_with_the_most_strips(prec, bits, ny, oracle_so, oracle_env, tmp_path):
+    oracle_env("dot2")
+    g, c = Engine(), Engine(oracle_so)
+    try:
+        _check(g, c, "ppcg", prec, bits, 62 * 129 + 1, ny, [RUNS["ppcg"][5]] + MORE_PPCG, tmp_path)
+    finally:
+        g.finalize()
+        c.finalize()
+
+
 def test_mesh_too_wide_is_left_alone(tmp_path):
     g = Engine()
     try:
