@@ -25,7 +25,7 @@ import sys
 import pytest
 
 from conftest import REF_HIP, REF_ORACLE, REPO, run_in_dir
-from tealeaf_cuda_amd import Deck, StateSpec, parse_tea_out, random_layout, run_deck, standard_states
+from tealeaf_cuda_amd import Deck, Engine, StateSpec, parse_tea_out, random_layout, run_deck, standard_states
 
 pytestmark = pytest.mark.gpu
 
@@ -96,6 +96,32 @@ def test_production_shape_bitwise_in_passes(precision, oracle_so, driver_built, 
     at 4096^2."""
     monkeypatch.setenv("TEA_RESIDENT", "0")
     test_production_shape_bitwise(precision, oracle_so, driver_built, oracle_env, tmp_path)
+
+
+@pytest.mark.parametrize("refinement", ["reliable", "restart"])
+def test_one_cg_iteration_writes_no_owed_w(refinement, driver_built, monkeypatch, tmp_path):
+    """A refined PPCG solve after the first makes one CG iteration, then
+    switches: that iteration writes w, instead of owing it and having it formed
+    again (where PPCG iterations end the solve, they owe w as they always do)."""
+    print(f"[gpu configs] one CG iteration before the switch, {refinement}", flush=True)
+    monkeypatch.setenv("TEA_RESIDENT", "0")
+    path = Deck(x_cells=96, y_cells=80, end_step=3, solver="ppcg", preconditioner="jac_block", eps=1e-10,
+                ppcg_inner_steps=10, ch_cg_presteps=10, ch_cg_epslim=1e9, summary_frequency=0, inner_precision="fp32",
+                mixed_refinement=refinement, inner_eps=1e-5 if refinement == "restart" else None,
+                states=standard_states()).write(tmp_path / "tea.in")
+    eng, seen = Engine(), {}
+
+    def on_step(step):
+        if step == 1:
+            eng.profile_reset()
+            eng.profile_enable(True)
+        elif step == 3:
+            eng.profile_enable(False)
+            seen.update(eng.profile())
+
+    run_deck(path, on_step=on_step)
+    assert "k_cg_calc_ur_f32" in seen and "cg_begin_f32" not in seen, sorted(seen)
+    assert refinement == "restart" or "settle_w_f32" not in seen, sorted(seen)
 
 
 LAYOUT = [StateSpec(100.0, 0.0001), StateSpec(0.1, 25.0, "rectangle", 0.0, 1.0, 1.0, 2.0),
