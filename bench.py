@@ -96,6 +96,8 @@ COMPULSORY_BYTES = {
     "ppcg_end_rr_f32": 16, "ppcg_end_rr": 32,
     # the begin after it: p, z (utemp), Kx, Ky read; p' written
     "ppcg_begin_pw_f32": 20, "ppcg_begin_pw": 40,
+    # fused CG: begin (p, z, Kx, Ky read; p' written), ur (u, p', r, Kx, Ky read; u, r, z written)
+    "cg_begin_f32": 20, "cg_begin": 40, "cg_ur_f32": 32, "cg_ur": 64,
     # CG iteration kernels: w = Ap (p, Kx, Ky read; w written); u/r/z update (u, p, r, w, Kx, Ky read;
     # u, r, z written); p = z + beta p (z, p read; p written)
     "cg_calc_w_f32": 16, "cg_calc_w": 32,

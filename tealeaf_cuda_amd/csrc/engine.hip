@@ -2754,10 +2754,16 @@ EXPORT void tea_leaf_ppcg_calc_p_kernel_cuda_(double *beta)
 
 // ---- resident runs (no reference counterpart) ----------------------------------------
 //
-// Many iterations in one launch (resident.hpp) for every mesh whose fields fit
-// the chip (about 1500^2 cells in FP64, 2000^2 in FP32): a run wins from the
-// smallest to the largest of them (whole decks: 2.5 times at 10^2 cells, 4.8 at
-// 1000^2; at 1531 x 997, four strips per wave, PPCG 1.9 times).  TEA_RESIDENT=0
+// Many iterations in one launch (resident.hpp) for every mesh that plan_tiles
+// takes: bands of at most 62 columns, floor(compute units / bands) tiles in each,
+// a tile of at most 32 strips of 4 rows in FP64 and 64 in FP32.  On 256 compute
+// units that is up to 1408^2 and 1984^2, and 1531 x 997 or 8060 x 128 (256) as
+// well.  Why every one of them: against the separate kernels (whole decks,
+// squares of 100 to 1400 and 1980 and strips of 8 to 16384 rows, every solver
+// and preconditioner) a run won each time, CG 2.2 to 5.3 times, Chebyshev 1.4 to
+// 3.6, PPCG 1.5 to 3.6 in FP64 and 1.14 to 2.6 in FP32; least on 100^2 cells in
+// FP32 (1.43 for 1.65 ms) and, among the large, FP32 PPCG with block Jacobi at
+// 8 strips per wave (1980^2: 19.9 for 24.2 ms), which spills 176 registers.  TEA_RESIDENT=0
 // turns them off, and so does any switch that picks a form of the separate
 // kernels.
 namespace {

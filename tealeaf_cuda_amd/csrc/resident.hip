@@ -17,8 +17,8 @@ constexpr long long EXCHANGE_TICKS = 1000000000;  // 10 s
 // How long a wave waits (64 clocks each) before its first look for the other
 // workgroups' sums where it has nothing else to do meanwhile, and between two
 // looks: 255 workgroups reading the same lines hold up the stores they wait
-// for (an iteration of 1000^2 cells: 12.2 us without the waits and with one
-// copy of the sums, 10.0 with both, PREC_NONE, 6 strips in 4 waves).
+// for (a CG deck of 1000^2 cells, 879 iterations: 7.6 ms; without the first wait
+// 8.7, with one copy of the sums instead of eight 8.4, without both 9.9).
 constexpr int FIRST_LOOK = 24, NEXT_LOOK = 2;
 
 __device__ __forceinline__ word_t load_word(const word_t *p)
@@ -763,11 +763,13 @@ __global__ __launch_bounds__(RES_BLOCK, 2) void k_cg_resident(Tiles t, Fields<T>
 // them too (more would spill inside the inner steps, and a spill there costs
 // more than the reads).  An inner step is one neighbour exchange (no
 // all-reduce): bound by its latency on small meshes, by issue on the largest.
-// Measured, FP64, a deck's whole run with its CG steps and set-up, against the
-// separate passes: 512^2 block Jacobi, 10 inner steps 4.56 (11.11) ms; 1531 x
-// 997 jac_diag, halo depth 2, to the FP64 true residual 10.89 (20.65) ms (with
+// Measured, a deck's whole run with its CG steps and set-up, against the
+// separate passes: FP64, 512^2 block Jacobi, 10 inner steps 4.42 (10.50) ms; 1531
+// x 997 jac_diag, halo depth 2, to the FP64 true residual 10.64 (20.12) ms (with
 // selects per row instead of branches per strip 9% more).  There, four strips
-// per wave, two thirds of an inner step are issue and a fifth the exchange.
+// per wave, two thirds of an inner step are issue and a fifth the exchange, and
+// 86 registers spill (152 with block Jacobi: 1400^2 8.4 (15.9) ms).  FP32 block
+// Jacobi: 1000^2, 3 strips, 4.5 (8.3) ms; 1980^2, 8 strips, 19.9 (24.2) ms.
 template <typename T, int PREC, int S>
 __global__ __launch_bounds__(RES_BLOCK, 2) void k_ppcg_resident(Tiles t, Fields<T> f, Exchange x, int from_inner,
                                                                 int with_p, double beta_in, double rro,
